@@ -14,6 +14,7 @@
 // (mac2d/_triton_mg.py:7-75), so results are bit-identical to the
 // restatement in FP64 (compiled with -ffp-contract=off).
 #include "binshare.hpp"
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -375,330 +376,76 @@ int ch_prolong(const T* coarse, T* fine, const int64_t n[2], int periodic, hipSt
     return OK;
 }
 
+#include "channel_vcycle.hpp"
+
+template <class T>
+__global__ void __launch_bounds__(CHF_NT) chf_tile_kernel(afsi_mg2d_plan pl, int l, int chunk, bool up) {
+    __shared__ T box[2 * CHF_B * CHF_PITCH], tab[9];
+    if (pl.periodic) chf_tile<T, true>(pl, l, int(blockIdx.x), chunk, up, box, tab);
+    else chf_tile<T, false>(pl, l, int(blockIdx.x), chunk, up, box, tab);
+}
+
+template <class T, bool P>
+__global__ void __launch_bounds__(CHF_TAIL_NT) chf_tail_kernel(afsi_mg2d_plan pl, int l0, int cycles) {
+    extern __shared__ unsigned char raw[];
+    __shared__ ChfShared<T> sh;
+    chf_tail<T, P>(pl, l0, cycles, reinterpret_cast<T*>(raw), sh);
+}
+
+// x -= sum / count, the sum from `parts` partials (stride 4) in a fixed order.
+template <class T>
+__global__ void __launch_bounds__(CH_THREADS) ch_sub_partials_kernel(T* __restrict__ x, int count,
+                                                                     const double* __restrict__ partials, int parts) {
+    double v = 0.0;
+    for (int b = int(threadIdx.x) % WAVE; b < parts; b += WAVE) v += partials[4 * b];
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) v += __shfl_xor(v, dd, WAVE);
+    const T mean = T(v / double(count));
+    for (int i = blockIdx.x * CH_THREADS + threadIdx.x; i < count; i += gridDim.x * CH_THREADS) x[i] = x[i] - mean;
+}
+
+// tmp = rhs - A p and its [sum, squares, |.|, non-finite] per workgroup.
+template <class T, bool P, bool M>
+__global__ void __launch_bounds__(CH_THREADS) ch_residual_kernel(const T* __restrict__ p, const T* __restrict__ rhs,
+                                                                 T* __restrict__ out, Dim2 d, Coef2<T> k,
+                                                                 double* __restrict__ partials) {
+    __shared__ double red[4][CH_THREADS / WAVE];
+    const int n = d.nx * d.ny, per = (n + int(gridDim.x) - 1) / int(gridDim.x);
+    const int begin = int(blockIdx.x) * per, end = min(begin + per, n);
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int i = begin + int(threadIdx.x); i < end; i += CH_THREADS) {
+        const int x = i / d.ny, y = i - x * d.ny;
+        T c;
+        const T r = rhs[i] - ch_apply<T, P, M>(p, x, y, d, k, c);
+        out[i] = r;
+        const double a = double(r);
+        if (isfinite(a)) {
+            v[0] += a;
+            v[1] += a * a;
+            v[2] += fabs(a);
+        } else {
+            v[3] += 1.0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int dd = 32; dd >= 1; dd >>= 1) v[q] += __shfl_xor(v[q], dd, WAVE);
+        if (threadIdx.x % WAVE == 0) red[q][threadIdx.x / WAVE] = v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        double t = 0.0;
+        for (int w = 0; w < CH_THREADS / WAVE; ++w) t += red[threadIdx.x][w];
+        partials[4 * blockIdx.x + threadIdx.x] = t;
+    }
+}
+
 }  // namespace
 
-// ---- whole V-cycles in one workgroup ----------------------------------------
-// For grids up to CHB_MAX_CELLS cells the launches of a V-cycle (a few
-// microseconds each) cost more than their work. One 1024-thread workgroup
-// then runs `cycles` complete V-cycles: every phase of the multi-launch
-// driver below becomes a block-strided loop over the same cells with the
-// same per-cell expressions (ch_apply, ch_diag, ch_coarse_value; the coarse
-// product with one wave per row and the same lane order and xor butterfly),
-// separated by __syncthreads(), which orders the global-memory writes of one
-// phase before the reads of the next within the workgroup. Results are the
-// multi-launch driver's bit for bit, except the periodic mean removal, whose
-// sum is taken in the workgroup's own fixed order.
-constexpr int CHB_THREADS = 1024;
-constexpr int64_t CHB_MAX_CELLS = 256 * 64;  // measured crossover: 2.05 vs 3.02 ms at 256x64, 6.4 vs 3.6 ms at 512x128
-// A thread takes its cells of a phase in groups of CHB_ILP: every load of a
-// group is issued before any of its stores, so the global-memory latencies
-// of the group overlap (the compiler cannot move a load above a store to
-// another array it may alias). Within a phase no cell reads what another
-// cell of the phase writes (a colour reads only the other colour), so the
-// values are those of the one-cell-at-a-time loop.
-constexpr int CHB_ILP = 4;
-
+int launch_reduce_final(const double* partials, int64_t nparts, double* result, hipStream_t s);
 template <class T>
-__device__ void chb_remove_mean(T* x, int n, double* red) {
-    double v = 0.0;
-    for (int i = threadIdx.x; i < n; i += CHB_THREADS) v += double(x[i]);
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = CHB_THREADS / 2; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    const T mean = T(red[0] / double(n));
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += CHB_THREADS) x[i] = x[i] - mean;
-    __syncthreads();
-}
-
-template <class T, bool P, bool M>
-__device__ __forceinline__ void chb_smooth(const afsi_mg2d_plan& pl, int l, double* red) {
-    const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-    const Coef2<T> k = coef2_of<T>(pl.h2[l][0], pl.h2[l][1], pl.inv_h2[l][0], pl.inv_h2[l][1]);
-    T* p = static_cast<T*>(pl.p[l]);
-    const T* rhs = static_cast<const T*>(pl.rhs[l]);
-    const int n = d.nx * d.ny;
-    if (pl.smoother == 1) {
-        for (int it = 0; it < pl.nu; ++it)
-            for (int color = 0; color < 2; ++color) {
-                if (d.ny % 2 == 0) {
-                    const int hy = d.ny / 2, half = d.nx * hy;
-                    for (int e0 = threadIdx.x; e0 < half; e0 += CHB_THREADS * CHB_ILP) {
-                        T val[CHB_ILP];
-                        int at[CHB_ILP];
-#pragma unroll
-                        for (int g = 0; g < CHB_ILP; ++g) {
-                            const int e = e0 + g * CHB_THREADS;
-                            at[g] = -1;
-                            if (e >= half) continue;
-                            const int x = e / hy, y = 2 * (e - x * hy) + ((x + color) & 1);
-                            const int i = x * d.ny + y;
-                            T c;
-                            const T r = rhs[i] - ch_apply<T, P, M>(p, x, y, d, k, c);
-                            val[g] = c + r / ch_diag<T, P>(x, y, d, k);
-                            at[g] = i;
-                        }
-#pragma unroll
-                        for (int g = 0; g < CHB_ILP; ++g)
-                            if (at[g] >= 0) p[at[g]] = val[g];
-                    }
-                } else {
-                    for (int i0 = threadIdx.x; i0 < n; i0 += CHB_THREADS * CHB_ILP) {
-                        T val[CHB_ILP];
-                        int at[CHB_ILP];
-#pragma unroll
-                        for (int g = 0; g < CHB_ILP; ++g) {
-                            const int i = i0 + g * CHB_THREADS;
-                            at[g] = -1;
-                            if (i >= n) continue;
-                            const int x = i / d.ny, y = i - x * d.ny;
-                            if (((x + y) & 1) != color) continue;
-                            T c;
-                            const T r = rhs[i] - ch_apply<T, P, M>(p, x, y, d, k, c);
-                            val[g] = c + r / ch_diag<T, P>(x, y, d, k);
-                            at[g] = i;
-                        }
-#pragma unroll
-                        for (int g = 0; g < CHB_ILP; ++g)
-                            if (at[g] >= 0) p[at[g]] = val[g];
-                    }
-                }
-                __syncthreads();
-            }
-    } else {
-        T* a = p;
-        T* b = static_cast<T*>(pl.tmp[l]);
-        const T omega = T(pl.omega);
-        for (int it = 0; it < pl.nu; ++it) {
-            for (int i0 = threadIdx.x; i0 < n; i0 += CHB_THREADS * CHB_ILP) {
-                T val[CHB_ILP];
-#pragma unroll
-                for (int g = 0; g < CHB_ILP; ++g) {
-                    const int i = i0 + g * CHB_THREADS;
-                    if (i >= n) continue;
-                    const int x = i / d.ny, y = i - x * d.ny;
-                    T c;
-                    const T r = rhs[i] - ch_apply<T, P, M>(a, x, y, d, k, c);
-                    val[g] = c + (omega * r) / ch_diag<T, P>(x, y, d, k);
-                }
-#pragma unroll
-                for (int g = 0; g < CHB_ILP; ++g)
-                    if (i0 + g * CHB_THREADS < n) b[i0 + g * CHB_THREADS] = val[g];
-            }
-            __syncthreads();
-            T* t = a; a = b; b = t;
-        }
-        if (a != p) {
-            for (int i = threadIdx.x; i < n; i += CHB_THREADS) p[i] = a[i];
-            __syncthreads();
-        }
-    }
-    if (P) chb_remove_mean(p, n, red);
-}
-
-// Residual restriction of level l into rhs[l + 1] (the multi-launch
-// ch_residual_restrict_kernel's expressions).
-template <class T, bool P, bool M>
-__device__ __forceinline__ void chb_restrict(const afsi_mg2d_plan& pl, int l) {
-    const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-    const Coef2<T> k = coef2_of<T>(pl.h2[l][0], pl.h2[l][1], 0.0, 0.0);
-    const T* p = static_cast<const T*>(pl.p[l]);
-    const T* rhs = static_cast<const T*>(pl.rhs[l]);
-    T* coarse = static_cast<T*>(pl.rhs[l + 1]);
-    const int cy = d.ny / 2, nc = (d.nx / 2) * cy;
-    for (int i0 = threadIdx.x; i0 < nc; i0 += CHB_THREADS * CHB_ILP) {
-        T val[CHB_ILP];
-#pragma unroll
-        for (int g = 0; g < CHB_ILP; ++g) {
-            const int i = i0 + g * CHB_THREADS;
-            if (i >= nc) continue;
-            const int X = i / cy, Y = i - X * cy;
-            const int x = 2 * X, y = 2 * Y, j = x * d.ny + y;
-            T c;
-            const T r00 = rhs[j] - ch_apply<T, P, M>(p, x, y, d, k, c);
-            const T r01 = rhs[j + 1] - ch_apply<T, P, M>(p, x, y + 1, d, k, c);
-            const T r10 = rhs[j + d.ny] - ch_apply<T, P, M>(p, x + 1, y, d, k, c);
-            const T r11 = rhs[j + d.ny + 1] - ch_apply<T, P, M>(p, x + 1, y + 1, d, k, c);
-            val[g] = (((r00 + r01) + r10) + r11) * T(0.25);
-        }
-#pragma unroll
-        for (int g = 0; g < CHB_ILP; ++g)
-            if (i0 + g * CHB_THREADS < nc) coarse[i0 + g * CHB_THREADS] = val[g];
-    }
-}
-
-// Whether level l's spacings are powers of two (exact multiplications).
-__device__ inline bool chb_exact(const afsi_mg2d_plan& pl, int l) {
-    return exact_recip(pl.h2[l][0]) != 0.0 && exact_recip(pl.h2[l][1]) != 0.0;
-}
-
-template <class T, bool P>
-__device__ __forceinline__ void chb_smooth_level(const afsi_mg2d_plan& pl, int l, double* red) {
-    if (chb_exact(pl, l)) chb_smooth<T, P, true>(pl, l, red);
-    else chb_smooth<T, P, false>(pl, l, red);
-}
-
-// `cycles` V-cycles of levels l0..last (l0 > 0: the lower part of a cycle
-// whose levels above l0 run as batched launches).
-template <class T, bool P>
-__device__ __forceinline__ void chb_cycles(const afsi_mg2d_plan& pl, int cycles, double* red, int l0 = 0) {
-    const int last = pl.levels - 1;
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-    for (int cyc = 0; cyc < cycles; ++cyc) {
-        for (int l = l0; l < last; ++l) {
-            chb_smooth_level<T, P>(pl, l, red);
-            if (chb_exact(pl, l)) chb_restrict<T, P, true>(pl, l);
-            else chb_restrict<T, P, false>(pl, l);
-            const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-            T* coarse = static_cast<T*>(pl.rhs[l + 1]);
-            const int cy = d.ny / 2, nc = (d.nx / 2) * cy;
-            __syncthreads();
-            if (P) chb_remove_mean(coarse, nc, red);
-            T* pc = static_cast<T*>(pl.p[l + 1]);
-            for (int i = threadIdx.x; i < nc; i += CHB_THREADS) pc[i] = T(0);
-            __syncthreads();
-        }
-        {   // coarsest: p = inverse * rhs, one wave per row
-            const int m = int(pl.coarse_cells);
-            const T* A = static_cast<const T*>(pl.coarse_inverse);
-            const T* xv = static_cast<const T*>(pl.rhs[last]);
-            T* y = static_cast<T*>(pl.p[last]);
-            for (int r = wave; r < m; r += CHB_THREADS / WAVE) {
-                T acc = T(0);
-                for (int c = lane; c < m; c += WAVE) acc += A[int64_t(r) * m + c] * xv[c];
-#pragma unroll
-                for (int dd = 32; dd >= 1; dd >>= 1) acc += __shfl_xor(acc, dd, WAVE);
-                if (lane == 0) y[r] = acc;
-            }
-            __syncthreads();
-            if (P) chb_remove_mean(y, m, red);
-        }
-        for (int l = last - 1; l >= l0; --l) {
-            const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-            const T* coarse = static_cast<const T*>(pl.p[l + 1]);
-            T* fine = static_cast<T*>(pl.p[l]);
-            const int n = d.nx * d.ny, NX = d.nx / 2, NY = d.ny / 2;
-            for (int i0 = threadIdx.x; i0 < n; i0 += CHB_THREADS * CHB_ILP) {
-                T val[CHB_ILP];
-#pragma unroll
-                for (int g = 0; g < CHB_ILP; ++g) {
-                    const int i = i0 + g * CHB_THREADS;
-                    if (i >= n) continue;
-                    const int x = i / d.ny, y = i - x * d.ny;
-                    const int ax = x / 2 - 1 + (x & 1), ay = y / 2 - 1 + (y & 1);
-                    const T wx = (x & 1) ? T(0.25) : T(0.75), wy = (y & 1) ? T(0.25) : T(0.75);
-                    const T c00 = ch_coarse_value<T, P>(coarse, ax, ay, NX, NY);
-                    const T c01 = ch_coarse_value<T, P>(coarse, ax, ay + 1, NX, NY);
-                    const T c10 = ch_coarse_value<T, P>(coarse, ax + 1, ay, NX, NY);
-                    const T c11 = ch_coarse_value<T, P>(coarse, ax + 1, ay + 1, NX, NY);
-                    const T v = (c00 * (T(1) - wy) + c01 * wy) * (T(1) - wx) + (c10 * (T(1) - wy) + c11 * wy) * wx;
-                    val[g] = fine[i] + v;
-                }
-#pragma unroll
-                for (int g = 0; g < CHB_ILP; ++g)
-                    if (i0 + g * CHB_THREADS < n) fine[i0 + g * CHB_THREADS] = val[g];
-            }
-            __syncthreads();
-            chb_smooth_level<T, P>(pl, l, red);
-        }
-    }
-}
-
-template <class T, bool P>
-__global__ void __launch_bounds__(CHB_THREADS) ch_block_cycles_kernel(afsi_mg2d_plan pl, int cycles) {
-    __shared__ double red[CHB_THREADS];
-    chb_cycles<T, P>(pl, cycles, red);
-}
-
-// ---- native V-cycle driver ---------------------------------------------------
-
-template <class T>
-struct ChannelRunner {
-    const afsi_mg2d_plan& pl;
-    hipStream_t s;
-
-    T* P(int l) const { return static_cast<T*>(pl.p[l]); }
-    T* R(int l) const { return static_cast<T*>(pl.rhs[l]); }
-    T* W(int l) const { return static_cast<T*>(pl.tmp[l]); }
-    int64_t cells(int l) const { return pl.n[l][0] * pl.n[l][1]; }
-
-    int remove_mean(T* x, int64_t count) const;
-
-    int smooth(int l) const {
-        if (pl.smoother == 1) {
-            for (int k = 0; k < pl.nu; ++k)
-                for (int color = 0; color < 2; ++color)
-                    if (int r = ch_rbgs<T>(P(l), R(l), pl.n[l], pl.h2[l], pl.inv_h2[l], color,
-                                           pl.periodic, s))
-                        return r;
-        } else {
-            T* a = P(l);
-            T* b = W(l);
-            for (int k = 0; k < pl.nu; ++k) {
-                if (int r = ch_stencil<T, 1>(a, R(l), b, pl.n[l], pl.h2[l], pl.inv_h2[l], pl.omega,
-                                             pl.periodic, s))
-                    return r;
-                T* t = a; a = b; b = t;
-            }
-            if (a != P(l))
-                AFSI_HIP(hipMemcpyAsync(P(l), a, size_t(cells(l)) * sizeof(T),
-                                        hipMemcpyDeviceToDevice, s));
-        }
-        return pl.periodic ? remove_mean(P(l), cells(l)) : OK;
-    }
-
-    int cycle(int l) const {
-        const int last = pl.levels - 1;
-        if (l == last) {
-            if (int r = dense_matvec(R(l), P(l))) return r;
-            return pl.periodic ? remove_mean(P(l), cells(l)) : OK;
-        }
-        if (int r = smooth(l)) return r;
-        if (int r = ch_residual_restrict<T>(P(l), R(l), R(l + 1), pl.n[l], pl.h2[l], pl.periodic, s))
-            return r;
-        if (pl.periodic)
-            if (int r = remove_mean(R(l + 1), cells(l + 1))) return r;
-        if (int r = fill(P(l + 1), cells(l + 1))) return r;
-        if (int r = cycle(l + 1)) return r;
-        if (int r = ch_prolong<T>(P(l + 1), P(l), pl.n[l], pl.periodic, s)) return r;
-        return smooth(l);
-    }
-
-    int dense_matvec(const T* x, T* y) const;
-    int fill(T* x, int64_t count) const;
-};
-
-template <>
-int ChannelRunner<double>::remove_mean(double* x, int64_t count) const {
-    if (int r = afsi_reduce_f64(x, count, pl.reduce_partials, pl.reduce_result, s)) return r;
-    return afsi_sub_mean_f64(x, count, pl.reduce_result, s);
-}
-template <>
-int ChannelRunner<float>::remove_mean(float* x, int64_t count) const {
-    if (int r = afsi_reduce_f32(x, count, pl.reduce_partials, pl.reduce_result, s)) return r;
-    return afsi_sub_mean_f32(x, count, pl.reduce_result, s);
-}
-template <>
-int ChannelRunner<double>::dense_matvec(const double* x, double* y) const {
-    return afsi_dense_matvec_f64(static_cast<const double*>(pl.coarse_inverse), x, y,
-                                 pl.coarse_cells, s);
-}
-template <>
-int ChannelRunner<float>::dense_matvec(const float* x, float* y) const {
-    return afsi_dense_matvec_f32(static_cast<const float*>(pl.coarse_inverse), x, y,
-                                 pl.coarse_cells, s);
-}
-template <>
-int ChannelRunner<double>::fill(double* x, int64_t count) const {
-    return afsi_fill_f64(x, count, 0.0, s);
-}
-template <>
-int ChannelRunner<float>::fill(float* x, int64_t count) const {
-    return afsi_fill_f32(x, count, 0.0, s);
-}
+int launch_reduce_partials(const T* x, int64_t count, double* partials, hipStream_t s);
 
 template <class T>
 static int channel_check(const afsi_mg2d_plan* pl) {
@@ -721,19 +468,52 @@ static int channel_check(const afsi_mg2d_plan* pl) {
 }
 
 template <class T>
+static int channel_tail(const afsi_mg2d_plan& pl, int l0, int cycles, size_t bytes, hipStream_t s) {
+    const void* fn = pl.periodic ? reinterpret_cast<const void*>(chf_tail_kernel<T, true>)
+                                 : reinterpret_cast<const void*>(chf_tail_kernel<T, false>);
+    if (int r = dynamic_lds(fn, bytes)) return r;
+    if (pl.periodic) chf_tail_kernel<T, true><<<1, CHF_TAIL_NT, bytes, s>>>(pl, l0, cycles);
+    else chf_tail_kernel<T, false><<<1, CHF_TAIL_NT, bytes, s>>>(pl, l0, cycles);
+    AFSI_LAUNCH_CHECK();
+    return OK;
+}
+
+// V-cycles: the levels whose hierarchy does not fit one workgroup's LDS
+// (chf_split) as tiled launches, one per smoothing stage of up to CHF_MAX
+// phases, the rest in the tail. Measured per red-black V(2,2) cycle (FP64,
+// periodic, kernel time): 256x64 32 us (two tile launches of 5.4 us around a
+// 21.7 us tail) against 166 us with every phase on global memory in one
+// workgroup; 128x32 whole in the tail 16.4 us against 90 us. Jacobi V(4,4)
+// 512x128: 53 us in five launches against 135 us in 52. The line between
+// the two forms is the LDS: a level that fits costs 3-8 us in the tail, which
+// is less than two launches and their gaps.
+template <class T>
 static int channel_cycles(const afsi_mg2d_plan* pl, int32_t cycles, void* stream) {
     if (int r = channel_check<T>(pl)) return r;
     AFSI_REQUIRE(cycles >= 0, "negative cycle count");
-    if (pl->n[0][0] * pl->n[0][1] <= CHB_MAX_CELLS) {
-        if (cycles == 0) return OK;
-        if (pl->periodic) ch_block_cycles_kernel<T, true><<<1, CHB_THREADS, 0, hipStream_t(stream)>>>(*pl, cycles);
-        else ch_block_cycles_kernel<T, false><<<1, CHB_THREADS, 0, hipStream_t(stream)>>>(*pl, cycles);
+    if (cycles == 0) return OK;
+    const hipStream_t s = hipStream_t(stream);
+    size_t bytes = 0;
+    const int l0 = chf_split(*pl, sizeof(T), &bytes);
+    if (l0 == 0) return channel_tail<T>(*pl, 0, cycles, bytes, s);
+    const int chunks = chf_chunks(*pl);
+    const auto level = [&](int l, bool up) {
+        for (int c = 0; c < chunks; ++c)
+            chf_tile_kernel<T><<<unsigned(chf_tiles(*pl, l)), CHF_NT, 0, s>>>(*pl, l, c, up);
+    };
+    for (int c = 0; c < cycles; ++c) {
+        for (int l = 0; l < l0; ++l) level(l, false);
+        if (int r = channel_tail<T>(*pl, l0, 1, bytes, s)) return r;
+        for (int l = l0 - 1; l >= 0; --l) level(l, true);
         AFSI_LAUNCH_CHECK();
-        return OK;
     }
-    const ChannelRunner<T> run{*pl, hipStream_t(stream)};
-    for (int c = 0; c < cycles; ++c)
-        if (int r = run.cycle(0)) return r;
+    if (!pl->periodic) return OK;
+    const int64_t count = pl->n[0][0] * pl->n[0][1], parts = afsi_reduce_partials(count);
+    T* p = static_cast<T*>(pl->p[0]);
+    if (int r = launch_reduce_partials(p, count, pl->reduce_partials, s)) return r;
+    ch_sub_partials_kernel<T><<<grid_for(count, CH_THREADS, 1024), CH_THREADS, 0, s>>>(p, int(count),
+                                                                                     pl->reduce_partials, int(parts));
+    AFSI_LAUNCH_CHECK();
     return OK;
 }
 
@@ -741,15 +521,20 @@ template <class T>
 static int channel_residual(const afsi_mg2d_plan* pl, void* stream) {
     if (int r = channel_check<T>(pl)) return r;
     const hipStream_t s = hipStream_t(stream);
+    const T *p = static_cast<const T*>(pl->p[0]), *rhs = static_cast<const T*>(pl->rhs[0]);
     T* tmp = static_cast<T*>(pl->tmp[0]);
-    if (int r = ch_stencil<T, 0>(static_cast<const T*>(pl->p[0]), static_cast<const T*>(pl->rhs[0]),
-                                 tmp, pl->n[0], pl->h2[0], nullptr, 0.0, pl->periodic, s))
-        return r;
-    const int64_t count = pl->n[0][0] * pl->n[0][1];
-    if constexpr (sizeof(T) == 8)
-        return afsi_reduce_f64(tmp, count, pl->reduce_partials, pl->reduce_result, s);
-    else
-        return afsi_reduce_f32(tmp, count, pl->reduce_partials, pl->reduce_result, s);
+    const Dim2 d{int(pl->n[0][0]), int(pl->n[0][1])};
+    const Coef2<T> k = coef2<T>(pl->h2[0], nullptr);
+    const int64_t parts = afsi_reduce_partials(int64_t(d.nx) * d.ny);
+    const unsigned g = unsigned(parts);
+    double* out = pl->reduce_partials;
+    const bool m = k.exact();
+    if (pl->periodic && m) ch_residual_kernel<T, true, true><<<g, CH_THREADS, 0, s>>>(p, rhs, tmp, d, k, out);
+    else if (pl->periodic) ch_residual_kernel<T, true, false><<<g, CH_THREADS, 0, s>>>(p, rhs, tmp, d, k, out);
+    else if (m) ch_residual_kernel<T, false, true><<<g, CH_THREADS, 0, s>>>(p, rhs, tmp, d, k, out);
+    else ch_residual_kernel<T, false, false><<<g, CH_THREADS, 0, s>>>(p, rhs, tmp, d, k, out);
+    AFSI_LAUNCH_CHECK();
+    return launch_reduce_final(out, parts, pl->reduce_result, s);
 }
 
 }  // namespace afsi
@@ -1197,49 +982,10 @@ __global__ void __launch_bounds__(CH_THREADS) chb_correct_kernel(const ChbDesc* 
     }
 }
 
-// One workgroup per active instance: `cycles` V-cycles (ch_block_cycles).
-// One instantiation per boundary type (each holds one inlined V-cycle, so
-// the register budget of 1024 threads is not shared by two); workgroups of
-// the other type return at once, and so do instances whose upper levels run
-// as batched launches (split[i] > 0).
-template <bool P>
-__global__ void __launch_bounds__(CHB_THREADS) chb_cycles_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                                 const int32_t* __restrict__ split,
-                                                                 const int32_t* __restrict__ active, int cycles) {
-    __shared__ double red[CHB_THREADS];
-    const afsi_mg2d_plan& pl = plans[blockIdx.x];
-    if ((active && !active[blockIdx.x]) || (pl.periodic != 0) != P || split[blockIdx.x] > 0) return;
-    chb_cycles<double, P>(pl, cycles, red);
-}
-
-// The lower part (levels split[i]..last) of one V-cycle of every active
-// instance with split[i] > 0.
-template <bool P>
-__global__ void __launch_bounds__(CHB_THREADS) chb_tail_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                               const int32_t* __restrict__ split,
-                                                               const int32_t* __restrict__ active) {
-    __shared__ double red[CHB_THREADS];
-    const afsi_mg2d_plan& pl = plans[blockIdx.x];
-    const int l0 = split[blockIdx.x];
-    if ((active && !active[blockIdx.x]) || (pl.periodic != 0) != P || l0 <= 0) return;
-    chb_cycles<double, P>(pl, 1, red, l0);
-}
-
-// ---- upper levels of large instances as batched launches ---------------------
-// A level with more than MLB_MIN_CELLS cells (RBGS instances) would keep one
-// CU busy for hundreds of microseconds per cycle in the one-workgroup kernel:
-// its FP64 stencil work is issued by that one CU. Such levels run instead as
-// one launch per phase over every instance that has them, MLB_CHUNK cells of
-// one instance per workgroup, with the per-cell expressions of the
-// one-workgroup kernel (so smoothing, restriction and prolongation give the
-// same values). Only the periodic mean removal sums in another fixed order:
-// per-workgroup partial sums, then the instance's partials in workgroup
-// order. Level l's work list holds the instances whose first split[i]
-// levels include l; the levels below run in chb_tail_kernel.
-constexpr int MLB_THREADS = 256;
-constexpr int MLB_CHUNK = 2048;           // level-l cells per workgroup
-constexpr int64_t MLB_MIN_CELLS = 4096;
-
+// ---- V-cycles of many instances -----------------------------------------------
+// The launches of channel_cycles over every instance that has the level: a
+// work list per level holds the instances with their first tile, and the
+// tails run one workgroup per instance.
 struct MlbEntry {
     int32_t inst, block_begin;
 };
@@ -1254,210 +1000,83 @@ __device__ inline MlbEntry mlb_find(const MlbEntry* __restrict__ list, int n) {
     return list[lo];
 }
 
-template <bool P, bool M>
-__device__ __forceinline__ void mlb_smooth_chunk(const afsi_mg2d_plan& pl, int l, int chunk, int color) {
-    const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-    const Coef2<double> k = coef2_of<double>(pl.h2[l][0], pl.h2[l][1], pl.inv_h2[l][0], pl.inv_h2[l][1]);
-    double* p = static_cast<double*>(pl.p[l]);
-    const double* rhs = static_cast<const double*>(pl.rhs[l]);
-    const int hy = d.ny / 2, half = d.nx * hy;
-    constexpr int G = MLB_CHUNK / 2 / MLB_THREADS;
-    const int e0 = chunk * (MLB_CHUNK / 2) + int(threadIdx.x);
-    double val[G];
-    int at[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int e = e0 + g * MLB_THREADS;
-        at[g] = -1;
-        if (e >= half) continue;
-        const int x = e / hy, y = 2 * (e - x * hy) + ((x + color) & 1);
-        const int i = x * d.ny + y;
-        double c;
-        const double r = rhs[i] - ch_apply<double, P, M>(p, x, y, d, k, c);
-        val[g] = c + r / ch_diag<double, P>(x, y, d, k);
-        at[g] = i;
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-        if (at[g] >= 0) p[at[g]] = val[g];
-}
-
-// One colour of red-black iteration `it` on level l (instances with
-// pl.nu <= it skip it).
-__global__ void __launch_bounds__(MLB_THREADS) mlb_smooth_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                                 const MlbEntry* __restrict__ list, int n, int l,
-                                                                 int it, int color,
-                                                                 const int32_t* __restrict__ active) {
+__global__ void __launch_bounds__(CHF_NT) chf_tile_batch_kernel(const afsi_mg2d_plan* __restrict__ plans,
+                                                                const MlbEntry* __restrict__ list, int n, int l,
+                                                                int chunk, bool up,
+                                                                const int32_t* __restrict__ active) {
+    __shared__ double box[2 * CHF_B * CHF_PITCH], tab[9];
     const MlbEntry e = mlb_find(list, n);
     const afsi_mg2d_plan& pl = plans[e.inst];
-    if ((active && !active[e.inst]) || it >= pl.nu) return;
-    const int chunk = int(blockIdx.x) - e.block_begin;
-    const bool m = chb_exact(pl, l);
-    if (pl.periodic) {
-        if (m) mlb_smooth_chunk<true, true>(pl, l, chunk, color);
-        else mlb_smooth_chunk<true, false>(pl, l, chunk, color);
-    } else {
-        if (m) mlb_smooth_chunk<false, true>(pl, l, chunk, color);
-        else mlb_smooth_chunk<false, false>(pl, l, chunk, color);
-    }
+    if ((active && !active[e.inst]) || chunk >= chf_chunks(pl)) return;
+    const int tile = int(blockIdx.x) - e.block_begin;
+    if (pl.periodic) chf_tile<double, true>(pl, l, tile, chunk, up, box, tab);
+    else chf_tile<double, false>(pl, l, tile, chunk, up, box, tab);
 }
 
-// The range of a chunk of level l in the array being averaged: p[l]
-// (coarse == 0, MLB_CHUNK cells) or rhs[l + 1] (coarse == 1, a quarter).
-__device__ inline void mlb_mean_range(const afsi_mg2d_plan& pl, int l, int coarse, int chunk, double*& x,
-                                      int& begin, int& end, int& count) {
-    const int cells = int(pl.n[l][0] * pl.n[l][1]);
-    const int per = coarse ? MLB_CHUNK / 4 : MLB_CHUNK;
-    count = coarse ? cells / 4 : cells;
-    x = static_cast<double*>(coarse ? pl.rhs[l + 1] : pl.p[l]);
-    begin = chunk * per;
-    end = begin + per < count ? begin + per : count;
+// Tails of the instances of one boundary type: those that start at level 0
+// (whole: `cycles` whole V-cycles) or below.
+template <bool P>
+__global__ void __launch_bounds__(CHF_TAIL_NT) chf_tail_batch_kernel(const afsi_mg2d_plan* __restrict__ plans,
+                                                                     const int32_t* __restrict__ split,
+                                                                     const int32_t* __restrict__ active, bool whole,
+                                                                     int cycles) {
+    extern __shared__ unsigned char raw[];
+    __shared__ ChfShared<double> sh;
+    const afsi_mg2d_plan& pl = plans[blockIdx.x];
+    const int l0 = split[blockIdx.x];
+    if ((active && !active[blockIdx.x]) || (pl.periodic != 0) != P || (l0 == 0) != whole) return;
+    chf_tail<double, P>(pl, l0, cycles, reinterpret_cast<double*>(raw), sh);
 }
 
-// Partial sum of the chunk (periodic instances), in a fixed order.
+constexpr int MLB_THREADS = 256;
+constexpr int MLB_CHUNK = 2048;  // level-0 cells per workgroup of the reductions
+
+// Mean removal of p[0] after the cycles of periodic instances whose level 0
+// is tiled: partial sums per chunk, then the instance's partials in chunk order.
 __global__ void __launch_bounds__(MLB_THREADS) mlb_sum_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                              const MlbEntry* __restrict__ list, int n, int l,
-                                                              int coarse, const int32_t* __restrict__ active,
+                                                              const MlbEntry* __restrict__ list, int n,
+                                                              const int32_t* __restrict__ split,
+                                                              const int32_t* __restrict__ active,
                                                               double* __restrict__ partials) {
-    __shared__ double red[MLB_THREADS];
+    __shared__ double red[MLB_THREADS / WAVE];
     const MlbEntry e = mlb_find(list, n);
     const afsi_mg2d_plan& pl = plans[e.inst];
-    if ((active && !active[e.inst]) || !pl.periodic) return;
-    double* x;
-    int begin, end, count;
-    mlb_mean_range(pl, l, coarse, int(blockIdx.x) - e.block_begin, x, begin, end, count);
+    if ((active && !active[e.inst]) || !pl.periodic || split[e.inst] == 0) return;
+    const double* x = static_cast<const double*>(pl.p[0]);
+    const int count = int(pl.n[0][0] * pl.n[0][1]);
+    const int begin = (int(blockIdx.x) - e.block_begin) * MLB_CHUNK, end = min(begin + MLB_CHUNK, count);
     double v = 0.0;
     for (int i = begin + int(threadIdx.x); i < end; i += MLB_THREADS) v += x[i];
-    red[threadIdx.x] = v;
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) v += __shfl_xor(v, dd, WAVE);
+    if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE] = v;
     __syncthreads();
-    for (int w = MLB_THREADS / 2; w > 0; w >>= 1) {
-        if (int(threadIdx.x) < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < MLB_THREADS / WAVE; ++w) t += red[w];
+        partials[blockIdx.x] = t;
     }
-    if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
 }
 
-// x -= mean, the mean from the instance's partials in workgroup order.
 __global__ void __launch_bounds__(MLB_THREADS) mlb_sub_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                              const MlbEntry* __restrict__ list, int n, int l,
-                                                              int coarse, const int32_t* __restrict__ active,
+                                                              const MlbEntry* __restrict__ list, int n,
+                                                              const int32_t* __restrict__ split,
+                                                              const int32_t* __restrict__ active,
                                                               const double* __restrict__ partials) {
-    __shared__ double total;
     const MlbEntry e = mlb_find(list, n);
     const afsi_mg2d_plan& pl = plans[e.inst];
-    if ((active && !active[e.inst]) || !pl.periodic) return;
-    double* x;
-    int begin, end, count;
-    mlb_mean_range(pl, l, coarse, int(blockIdx.x) - e.block_begin, x, begin, end, count);
-    if (threadIdx.x == 0) {
-        const int blocks = int((pl.n[l][0] * pl.n[l][1] + MLB_CHUNK - 1) / MLB_CHUNK);
-        double t = 0.0;
-        for (int b = 0; b < blocks; ++b) t += partials[e.block_begin + b];
-        total = t;
-    }
-    __syncthreads();
-    const double mean = total / double(count);
+    if ((active && !active[e.inst]) || !pl.periodic || split[e.inst] == 0) return;
+    double* x = static_cast<double*>(pl.p[0]);
+    const int count = int(pl.n[0][0] * pl.n[0][1]), blocks = (count + MLB_CHUNK - 1) / MLB_CHUNK;
+    const int begin = (int(blockIdx.x) - e.block_begin) * MLB_CHUNK, end = min(begin + MLB_CHUNK, count);
+    double v = 0.0;
+    for (int b = int(threadIdx.x) % WAVE; b < blocks; b += WAVE) v += partials[e.block_begin + b];
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) v += __shfl_xor(v, dd, WAVE);
+    const double mean = v / double(count);
     for (int i = begin + int(threadIdx.x); i < end; i += MLB_THREADS) x[i] = x[i] - mean;
 }
 
-template <bool P, bool M>
-__device__ __forceinline__ void mlb_restrict_chunk(const afsi_mg2d_plan& pl, int l, int chunk) {
-    const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-    const Coef2<double> k = coef2_of<double>(pl.h2[l][0], pl.h2[l][1], 0.0, 0.0);
-    const double* p = static_cast<const double*>(pl.p[l]);
-    const double* rhs = static_cast<const double*>(pl.rhs[l]);
-    double* coarse = static_cast<double*>(pl.rhs[l + 1]);
-    double* pc = static_cast<double*>(pl.p[l + 1]);
-    const int cy = d.ny / 2, nc = (d.nx / 2) * cy;
-    constexpr int G = MLB_CHUNK / 4 / MLB_THREADS;
-    const int i0 = chunk * (MLB_CHUNK / 4) + int(threadIdx.x);
-    double val[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int i = i0 + g * MLB_THREADS;
-        if (i >= nc) continue;
-        const int X = i / cy, Y = i - X * cy;
-        const int x = 2 * X, y = 2 * Y, j = x * d.ny + y;
-        double c;
-        const double r00 = rhs[j] - ch_apply<double, P, M>(p, x, y, d, k, c);
-        const double r01 = rhs[j + 1] - ch_apply<double, P, M>(p, x, y + 1, d, k, c);
-        const double r10 = rhs[j + d.ny] - ch_apply<double, P, M>(p, x + 1, y, d, k, c);
-        const double r11 = rhs[j + d.ny + 1] - ch_apply<double, P, M>(p, x + 1, y + 1, d, k, c);
-        val[g] = (((r00 + r01) + r10) + r11) * 0.25;
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int i = i0 + g * MLB_THREADS;
-        if (i < nc) {
-            coarse[i] = val[g];
-            pc[i] = 0.0;
-        }
-    }
-}
-
-// rhs[l + 1] = restricted residual of level l; p[l + 1] = 0.
-__global__ void __launch_bounds__(MLB_THREADS) mlb_restrict_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                                   const MlbEntry* __restrict__ list, int n, int l,
-                                                                   const int32_t* __restrict__ active) {
-    const MlbEntry e = mlb_find(list, n);
-    const afsi_mg2d_plan& pl = plans[e.inst];
-    if (active && !active[e.inst]) return;
-    const int chunk = int(blockIdx.x) - e.block_begin;
-    const bool m = chb_exact(pl, l);
-    if (pl.periodic) {
-        if (m) mlb_restrict_chunk<true, true>(pl, l, chunk);
-        else mlb_restrict_chunk<true, false>(pl, l, chunk);
-    } else {
-        if (m) mlb_restrict_chunk<false, true>(pl, l, chunk);
-        else mlb_restrict_chunk<false, false>(pl, l, chunk);
-    }
-}
-
-template <bool P>
-__device__ __forceinline__ void mlb_prolong_chunk(const afsi_mg2d_plan& pl, int l, int chunk) {
-    const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
-    const double* coarse = static_cast<const double*>(pl.p[l + 1]);
-    double* fine = static_cast<double*>(pl.p[l]);
-    const int n = d.nx * d.ny, NX = d.nx / 2, NY = d.ny / 2;
-    constexpr int G = MLB_CHUNK / MLB_THREADS;
-    const int i0 = chunk * MLB_CHUNK + int(threadIdx.x);
-    double val[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int i = i0 + g * MLB_THREADS;
-        if (i >= n) continue;
-        const int x = i / d.ny, y = i - x * d.ny;
-        const int ax = x / 2 - 1 + (x & 1), ay = y / 2 - 1 + (y & 1);
-        const double wx = (x & 1) ? 0.25 : 0.75, wy = (y & 1) ? 0.25 : 0.75;
-        const double c00 = ch_coarse_value<double, P>(coarse, ax, ay, NX, NY);
-        const double c01 = ch_coarse_value<double, P>(coarse, ax, ay + 1, NX, NY);
-        const double c10 = ch_coarse_value<double, P>(coarse, ax + 1, ay, NX, NY);
-        const double c11 = ch_coarse_value<double, P>(coarse, ax + 1, ay + 1, NX, NY);
-        const double v = (c00 * (1.0 - wy) + c01 * wy) * (1.0 - wx) + (c10 * (1.0 - wy) + c11 * wy) * wx;
-        val[g] = fine[i] + v;
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int i = i0 + g * MLB_THREADS;
-        if (i < n) fine[i] = val[g];
-    }
-}
-
-// p[l] += prolongation of p[l + 1].
-__global__ void __launch_bounds__(MLB_THREADS) mlb_prolong_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                                  const MlbEntry* __restrict__ list, int n, int l,
-                                                                  const int32_t* __restrict__ active) {
-    const MlbEntry e = mlb_find(list, n);
-    const afsi_mg2d_plan& pl = plans[e.inst];
-    if (active && !active[e.inst]) return;
-    const int chunk = int(blockIdx.x) - e.block_begin;
-    if (pl.periodic) mlb_prolong_chunk<true>(pl, l, chunk);
-    else mlb_prolong_chunk<false>(pl, l, chunk);
-}
-
-// One workgroup per instance: [sum, sum of squares, sum |.|, non-finite
-// count] of rhs[0] (which 0), p[0] (1) or rhs[0] - A p[0] (2), summed in a
-// fixed order; which 3/4: subtract the mean out[4i]/n from rhs[0]/p[0].
 // Value of cell i of level 0 for the statistics: rhs (which 0), p (1) or
 // the residual rhs - A p (2).
 __device__ inline double chb_stat_value(const afsi_mg2d_plan& pl, const Coef2<double>& k, bool m, int which,
@@ -1474,53 +1093,11 @@ __device__ inline double chb_stat_value(const afsi_mg2d_plan& pl, const Coef2<do
     return rhs[i] - (m ? ch_apply<double, false, true>(p, x, y, d, k, c) : ch_apply<double, false, false>(p, x, y, d, k, c));
 }
 
-__global__ void __launch_bounds__(CHB_THREADS) chb_stats_kernel(const afsi_mg2d_plan* __restrict__ plans,
-                                                                const int32_t* __restrict__ split, int which,
-                                                                double* __restrict__ out) {
-    __shared__ double red[4][CHB_THREADS];
-    if (split[blockIdx.x] > 0) return;  // level 0 is covered by mlb_stats_kernel
-    const afsi_mg2d_plan& pl = plans[blockIdx.x];
-    const Dim2 d{int(pl.n[0][0]), int(pl.n[0][1])};
-    const int n = d.nx * d.ny;
-    double* rhs = static_cast<double*>(pl.rhs[0]);
-    double* p = static_cast<double*>(pl.p[0]);
-    if (which >= 3) {  // mean removal: periodic channels only (the reference channel is non-singular)
-        if (!pl.periodic) return;
-        double* x = which == 3 ? rhs : p;
-        const double mean = out[4 * blockIdx.x] / double(n);
-        for (int i = threadIdx.x; i < n; i += CHB_THREADS) x[i] = x[i] - mean;
-        return;
-    }
-    const Coef2<double> k = coef2_of<double>(pl.h2[0][0], pl.h2[0][1], 0.0, 0.0);
-    const bool m = k.exact();
-    double s = 0.0, q = 0.0, a = 0.0, bad = 0.0;
-    for (int i = threadIdx.x; i < n; i += CHB_THREADS) {
-        const double v = chb_stat_value(pl, k, m, which, i);
-        if (isfinite(v)) {
-            s += v;
-            q += v * v;
-            a += fabs(v);
-        } else {
-            bad += 1.0;
-        }
-    }
-    red[0][threadIdx.x] = s;
-    red[1][threadIdx.x] = q;
-    red[2][threadIdx.x] = a;
-    red[3][threadIdx.x] = bad;
-    __syncthreads();
-    for (int w = CHB_THREADS / 2; w > 0; w >>= 1) {
-        if (int(threadIdx.x) < w)
-            for (int m = 0; m < 4; ++m) red[m][threadIdx.x] += red[m][threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x < 4) out[4 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
-}
-
-// The same statistics for instances whose level 0 runs as batched launches
-// (level-0 work list): partial [sum, squares, |.|, non-finite] per chunk in
-// a fixed order, then mlb_stats_final_kernel adds an instance's partials in
-// chunk order. which 3 / 4: subtract out[4i] / cells from the chunk.
+// Statistics of every instance: partial [sum, squares, |.|, non-finite] per
+// chunk of level 0 in a fixed order, then mlb_stats_final_kernel adds an
+// instance's partials in chunk order. which 3 / 4: subtract out[4i] / cells
+// from rhs[0] / p[0] of the periodic instances (the reference channel is
+// non-singular).
 __global__ void __launch_bounds__(MLB_THREADS) mlb_stats_kernel(const afsi_mg2d_plan* __restrict__ plans,
                                                                 const MlbEntry* __restrict__ list, int n, int which,
                                                                 double* __restrict__ partials,
@@ -1582,20 +1159,14 @@ struct ChbLayout {
     int64_t points = 0, nu = 0, nv = 0, cells = 0;
     size_t desc = 0, plans = 0, cell_begin = 0, split = 0, lists = 0, partials = 0, tiles = 0, total = 0;
     int64_t ntiles = 0;  // spread tiles over all instances and both components
-    // batched upper levels: levels 0..maxsplit-1 have work lists
-    int maxsplit = 0;
-    int count[AFSI_MG_MAX_LEVELS] = {}, blocks[AFSI_MG_MAX_LEVELS] = {}, max_nu[AFSI_MG_MAX_LEVELS] = {};
-    bool mean[AFSI_MG_MAX_LEVELS] = {};
-    bool whole_periodic = false, whole_closed = false, tail_periodic = false, tail_closed = false;
+    // tiled levels 0..maxsplit-1 have work lists; list AFSI_MG_MAX_LEVELS
+    // holds every instance's level-0 reduction chunks
+    int maxsplit = 0, reduce_blocks = 0;
+    int count[AFSI_MG_MAX_LEVELS] = {}, blocks[AFSI_MG_MAX_LEVELS] = {}, chunks[AFSI_MG_MAX_LEVELS] = {};
+    bool mean = false;
+    bool whole[2] = {false, false}, tail[2] = {false, false};  // by boundary type (1: periodic)
+    size_t tail_bytes = 0;
 };
-
-// Number of upper levels of an instance that run as batched launches.
-int mlb_split(const afsi_mg2d_plan& pl) {
-    if (pl.smoother != 1) return 0;
-    int s = 0;
-    while (s < pl.levels - 1 && pl.n[s][0] * pl.n[s][1] > MLB_MIN_CELLS && pl.n[s][1] % 2 == 0) ++s;
-    return s;
-}
 
 size_t chb_align(size_t b) { return (b + 255) & ~size_t(255); }
 
@@ -1637,11 +1208,13 @@ int chb_layout(const afsi_chb_batch* b, ChbLayout& L, std::vector<ChbDesc>* desc
             if (tiles) tiles->push_back(t);
             L.ntiles += int64_t(t.ntx) * t.nty;
         }
-        const int sp = mlb_split(pl);
+        size_t bytes = 0;
+        const int sp = chf_split(pl, sizeof(double), &bytes);
         if (splits) splits->push_back(sp);
         if (sp > L.maxsplit) L.maxsplit = sp;
-        if (sp == 0) (pl.periodic ? L.whole_periodic : L.whole_closed) = true;
-        else (pl.periodic ? L.tail_periodic : L.tail_closed) = true;
+        if (bytes > L.tail_bytes) L.tail_bytes = bytes;
+        (sp == 0 ? L.whole : L.tail)[pl.periodic ? 1 : 0] = true;
+        if (sp > 0 && pl.periodic) L.mean = true;
         L.points += it.points;
         L.nu += d.u_count;
         L.nv += d.v_count;
@@ -1650,30 +1223,34 @@ int chb_layout(const afsi_chb_batch* b, ChbLayout& L, std::vector<ChbDesc>* desc
     AFSI_REQUIRE(L.points < (int64_t(1) << 29) && L.nu < (int64_t(1) << 31) && L.nv < (int64_t(1) << 31) &&
                      L.ntiles < (int64_t(1) << 30),
                  "channel batch too large");
-    if (lists) lists->assign(size_t(AFSI_MG_MAX_LEVELS) * L.n, MlbEntry{0, 0});
-    int max_blocks = 1;
+    if (lists) lists->assign(size_t(AFSI_MG_MAX_LEVELS + 1) * L.n, MlbEntry{0, 0});
     for (int l = 0; l < L.maxsplit; ++l) {
         int64_t blocks = 0;
         for (int i = 0; i < L.n; ++i) {
             const afsi_mg2d_plan& pl = b->items[i].plan;
-            if (mlb_split(pl) <= l) continue;
+            if (chf_split(pl, sizeof(double), nullptr) <= l) continue;
             if (lists) (*lists)[size_t(l) * L.n + L.count[l]] = MlbEntry{i, int32_t(blocks)};
             ++L.count[l];
-            blocks += cdiv(pl.n[l][0] * pl.n[l][1], MLB_CHUNK);
-            if (pl.nu > L.max_nu[l]) L.max_nu[l] = pl.nu;
-            if (pl.periodic) L.mean[l] = true;
+            blocks += chf_tiles(pl, l);
+            L.chunks[l] = std::max(L.chunks[l], chf_chunks(pl));
         }
         AFSI_REQUIRE(blocks < (int64_t(1) << 30), "channel batch level too large");
         L.blocks[l] = int(blocks);
-        if (L.blocks[l] > max_blocks) max_blocks = L.blocks[l];
     }
+    int64_t blocks = 0;
+    for (int i = 0; i < L.n; ++i) {
+        if (lists) (*lists)[size_t(AFSI_MG_MAX_LEVELS) * L.n + i] = MlbEntry{i, int32_t(blocks)};
+        blocks += cdiv(b->items[i].plan.n[0][0] * b->items[i].plan.n[0][1], MLB_CHUNK);
+    }
+    AFSI_REQUIRE(blocks < (int64_t(1) << 30), "channel batch level too large");
+    L.reduce_blocks = int(blocks);
     size_t off = 0;
     L.desc = off; off = chb_align(off + size_t(L.n) * sizeof(ChbDesc));
     L.plans = off; off = chb_align(off + size_t(L.n) * sizeof(afsi_mg2d_plan));
     L.cell_begin = off; off = chb_align(off + size_t(L.n) * sizeof(int64_t));
     L.split = off; off = chb_align(off + size_t(L.n) * sizeof(int32_t));
-    L.lists = off; off = chb_align(off + size_t(AFSI_MG_MAX_LEVELS) * L.n * sizeof(MlbEntry));
-    L.partials = off; off = chb_align(off + 4 * size_t(max_blocks) * sizeof(double));
+    L.lists = off; off = chb_align(off + size_t(AFSI_MG_MAX_LEVELS + 1) * L.n * sizeof(MlbEntry));
+    L.partials = off; off = chb_align(off + 4 * size_t(L.reduce_blocks) * sizeof(double));
     L.tiles = off; off = chb_align(off + 2 * size_t(L.n) * sizeof(ChsTile));
     L.total = off;
     return OK;
@@ -1823,44 +1400,38 @@ int afsi_chb_cycles_f64(const afsi_chb_batch* batch, const int32_t* active, int3
     const hipStream_t s = hipStream_t(stream);
     const afsi_mg2d_plan* plans = chb_at<afsi_mg2d_plan>(batch, L.plans);
     const int32_t* split = chb_at<int32_t>(batch, L.split);
-    const unsigned n = unsigned(L.n);
-    // instances without batched levels: whole cycles, one workgroup each
-    if (L.whole_periodic) chb_cycles_kernel<true><<<n, CHB_THREADS, 0, s>>>(plans, split, active, cycles);
-    if (L.whole_closed) chb_cycles_kernel<false><<<n, CHB_THREADS, 0, s>>>(plans, split, active, cycles);
-    AFSI_LAUNCH_CHECK();
-    if (L.maxsplit == 0) return OK;
-    // the others: upper levels as batched launches around a one-workgroup tail
-    double* partials = chb_at<double>(batch, L.partials);
-    const auto list = [&](int l) { return chb_at<MlbEntry>(batch, L.lists) + size_t(l) * L.n; };
-    const auto smooth = [&](int l) {
-        for (int it = 0; it < L.max_nu[l]; ++it)
-            for (int color = 0; color < 2; ++color)
-                mlb_smooth_kernel<<<unsigned(L.blocks[l]), MLB_THREADS, 0, s>>>(plans, list(l), L.count[l], l, it,
-                                                                              color, active);
-    };
-    const auto remove_mean = [&](int l, int coarse) {
-        if (!L.mean[l]) return;
-        mlb_sum_kernel<<<unsigned(L.blocks[l]), MLB_THREADS, 0, s>>>(plans, list(l), L.count[l], l, coarse, active,
-                                                                      partials);
-        mlb_sub_kernel<<<unsigned(L.blocks[l]), MLB_THREADS, 0, s>>>(plans, list(l), L.count[l], l, coarse, active,
-                                                                      partials);
-    };
-    for (int c = 0; c < cycles; ++c) {
-        for (int l = 0; l < L.maxsplit; ++l) {
-            smooth(l);
-            remove_mean(l, 0);
-            mlb_restrict_kernel<<<unsigned(L.blocks[l]), MLB_THREADS, 0, s>>>(plans, list(l), L.count[l], l, active);
-            remove_mean(l, 1);
+    const auto tails = [&](bool whole, int count) -> int {
+        const bool* types = whole ? L.whole : L.tail;
+        if (types[0]) {
+            if (int r = dynamic_lds(reinterpret_cast<const void*>(chf_tail_batch_kernel<false>), L.tail_bytes)) return r;
+            chf_tail_batch_kernel<false><<<unsigned(L.n), CHF_TAIL_NT, L.tail_bytes, s>>>(plans, split, active, whole, count);
         }
-        if (L.tail_periodic) chb_tail_kernel<true><<<n, CHB_THREADS, 0, s>>>(plans, split, active);
-        if (L.tail_closed) chb_tail_kernel<false><<<n, CHB_THREADS, 0, s>>>(plans, split, active);
-        for (int l = L.maxsplit - 1; l >= 0; --l) {
-            mlb_prolong_kernel<<<unsigned(L.blocks[l]), MLB_THREADS, 0, s>>>(plans, list(l), L.count[l], l, active);
-            smooth(l);
-            remove_mean(l, 0);
+        if (types[1]) {
+            if (int r = dynamic_lds(reinterpret_cast<const void*>(chf_tail_batch_kernel<true>), L.tail_bytes)) return r;
+            chf_tail_batch_kernel<true><<<unsigned(L.n), CHF_TAIL_NT, L.tail_bytes, s>>>(plans, split, active, whole, count);
         }
         AFSI_LAUNCH_CHECK();
+        return OK;
+    };
+    if (int r = tails(true, cycles)) return r;
+    if (L.maxsplit == 0) return OK;
+    const auto list = [&](int l) { return chb_at<MlbEntry>(batch, L.lists) + size_t(l) * L.n; };
+    const auto level = [&](int l, bool up) {
+        for (int c = 0; c < L.chunks[l]; ++c)
+            chf_tile_batch_kernel<<<unsigned(L.blocks[l]), CHF_NT, 0, s>>>(plans, list(l), L.count[l], l, c, up, active);
+    };
+    for (int c = 0; c < cycles; ++c) {
+        for (int l = 0; l < L.maxsplit; ++l) level(l, false);
+        if (int r = tails(false, 1)) return r;
+        for (int l = L.maxsplit - 1; l >= 0; --l) level(l, true);
+        AFSI_LAUNCH_CHECK();
     }
+    if (!L.mean) return OK;
+    double* partials = chb_at<double>(batch, L.partials);
+    const MlbEntry* chunks = list(AFSI_MG_MAX_LEVELS);
+    mlb_sum_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, chunks, L.n, split, active, partials);
+    mlb_sub_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, chunks, L.n, split, active, partials);
+    AFSI_LAUNCH_CHECK();
     return OK;
 }
 
@@ -1870,17 +1441,12 @@ int afsi_chb_stats_f64(const afsi_chb_batch* batch, int which, double* out, void
     AFSI_REQUIRE(which >= 0 && which <= 4 && out, "invalid channel batch statistics request");
     const hipStream_t s = hipStream_t(stream);
     const afsi_mg2d_plan* plans = chb_at<afsi_mg2d_plan>(batch, L.plans);
-    chb_stats_kernel<<<unsigned(L.n), CHB_THREADS, 0, s>>>(plans, chb_at<int32_t>(batch, L.split), which, out);
+    const MlbEntry* list = chb_at<MlbEntry>(batch, L.lists) + size_t(AFSI_MG_MAX_LEVELS) * L.n;
+    double* partials = chb_at<double>(batch, L.partials);
+    mlb_stats_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, list, L.n, which, partials, out);
+    if (which < 3)
+        mlb_stats_final_kernel<<<unsigned(cdiv(4 * L.n, 256)), 256, 0, s>>>(plans, list, L.n, partials, out);
     AFSI_LAUNCH_CHECK();
-    if (L.maxsplit > 0) {
-        const MlbEntry* list = chb_at<MlbEntry>(batch, L.lists);
-        double* partials = chb_at<double>(batch, L.partials);
-        mlb_stats_kernel<<<unsigned(L.blocks[0]), MLB_THREADS, 0, s>>>(plans, list, L.count[0], which, partials, out);
-        if (which < 3)
-            mlb_stats_final_kernel<<<unsigned(cdiv(4 * L.count[0], 256)), 256, 0, s>>>(plans, list, L.count[0],
-                                                                                       partials, out);
-        AFSI_LAUNCH_CHECK();
-    }
     return OK;
 }
 

@@ -494,6 +494,17 @@ static int reduce(const T* x, int64_t count, double* partials, double* result, v
     return OK;
 }
 
+// The partials alone ([sum, squares, |.|, non-finite] each) of the
+// afsi_reduce_partials(count) workgroups of a reduction.
+template <class T>
+int launch_reduce_partials(const T* x, int64_t count, double* partials, hipStream_t s) {
+    reduce_partial_kernel<T><<<unsigned(reduce_blocks(count)), RED_THREADS, 0, s>>>(x, count, partials);
+    AFSI_LAUNCH_CHECK();
+    return OK;
+}
+template int launch_reduce_partials<double>(const double*, int64_t, double*, hipStream_t);
+template int launch_reduce_partials<float>(const float*, int64_t, double*, hipStream_t);
+
 int launch_reduce_final(const double* partials, int64_t nparts, double* result, hipStream_t s) {
     reduce_final_kernel<<<1, RED_THREADS, 0, s>>>(partials, nparts, result);
     AFSI_LAUNCH_CHECK();

@@ -1,0 +1,48 @@
+"""Channel V-cycles where the split between tiled launches and the one-
+workgroup tail, the tiles' edges and the phase chunks can go wrong: levels on
+either side of the tail's capacity (128x32, 160x32), extents that are no
+multiple of the 16-cell tile, sweeps that need two launches per stage, and a
+hierarchy of one level; against the oracle's cycle."""
+import numpy as np
+import pytest
+import torch
+
+from afsi_gpu_amd.mac import MGOptions
+from afsi_gpu_amd.mac2d import ChannelGrid, ChannelMultigrid
+from oracle import mac2d
+from oracle.mac3d import MGOptions as OOptions
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('periodic', [False, True], ids=['closed', 'periodic'])
+@pytest.mark.parametrize('smoother,nu', [('rbgs', 2), ('rbgs', 5), ('jacobi', 4), ('jacobi', 9)])
+@pytest.mark.parametrize('shape', [(24, 20), (128, 32), (160, 32), (192, 48), (72, 120), (512, 64)])
+def test_cycle_matches_oracle(gpu, shape, smoother, nu, periodic):
+    lengths = (4., 1.3)
+    grid = ChannelGrid(shape, lengths, periodic)
+    mg = ChannelMultigrid(grid, device=gpu, options=MGOptions(smooth=nu, smoother=smoother), backend='workspace')
+    ref = mac2d.ChannelMultigrid(shape, grid.spacing, OOptions(smooth=nu, smoother=smoother), periodic)
+    gen = np.random.default_rng(9)
+    p, rhs = gen.normal(size=shape), gen.normal(size=shape)
+    if periodic:
+        p, rhs = p - p.mean(), rhs - rhs.mean()
+    want = ref.cycle(0, p, rhs)
+    got = mg.cycle(torch.tensor(p, device=gpu), torch.tensor(rhs, device=gpu)).cpu().numpy()
+    # the cycle's own bound: about 50 FP64 roundings along any path of a contraction
+    assert np.linalg.norm(got - want) < 1e-12 * np.linalg.norm(want)
+    single = ChannelMultigrid(grid, device=gpu, dtype=torch.float32,
+                              options=MGOptions(smooth=nu, smoother=smoother), backend='workspace')
+    got = single.cycle(torch.tensor(p, device=gpu, dtype=torch.float32),
+                       torch.tensor(rhs, device=gpu, dtype=torch.float32)).double().cpu().numpy()
+    assert np.linalg.norm(got - want) < 1e-12 * 2. ** 29 * np.linalg.norm(want)  # the same bound in FP32
+
+
+def test_one_level(gpu):
+    grid = ChannelGrid((9, 5), (2., 1.))
+    mg = ChannelMultigrid(grid, device=gpu, backend='workspace')
+    rhs = np.random.default_rng(2).normal(size=(9, 5))
+    got = mg.cycle(torch.zeros((9, 5), device=gpu, dtype=torch.float64), torch.tensor(rhs, device=gpu)).cpu().numpy()
+    ref = mac2d.ChannelMultigrid((9, 5), grid.spacing, OOptions(), False)
+    want = ref.cycle(0, np.zeros((9, 5)), rhs)
+    assert np.linalg.norm(got - want) < 1e-12 * np.linalg.norm(want)
