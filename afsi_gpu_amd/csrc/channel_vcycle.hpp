@@ -79,9 +79,7 @@ struct ChfPair {
 
 template <class T>
 __device__ __forceinline__ T chf_update(const T* a, int at, int up, int down, T rhs, T inv, T wx, T wy) {
-    T s = __builtin_fma(wx, a[up] + a[down], rhs);
-    s = __builtin_fma(wy, a[at + 1] + a[at - 1], s);
-    return s * inv;
+    return fma_of(wy, a[at + 1] + a[at - 1], fma_of(wx, a[up] + a[down], rhs)) * inv;
 }
 
 // One launch's share of level l: tile `tile` of chunk `chunk` of the pre-

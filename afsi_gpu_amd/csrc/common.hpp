@@ -54,6 +54,10 @@ inline unsigned grid_for(int64_t work, int block, int64_t cap = 1 << 20) {
     return unsigned(g);
 }
 
+// a * b + c with one rounding, in the operands' type.
+__device__ inline float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ inline double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // Four Peskin weights for offsets 0..3 from f = s - base - 1 in [0,1):
 // |r| = 1+f, f, 1-f, 2-f all share the radical sqrt(1+4f-4f^2).
 template <class T>

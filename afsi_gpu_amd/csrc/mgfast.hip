@@ -51,7 +51,7 @@ struct W3 {
 // old + relax * (gs - old) when over-relaxed (relax is uniform per launch).
 template <class T>
 __device__ inline T rb_relax(const W3<T>& k, T old, T gs) {
-    return k.relax == T(1) ? gs : old + k.relax * (gs - old);
+    return k.relax == T(1) ? gs : fma_of(k.relax, gs - old, old);
 }
 
 __device__ inline int wrap32(int g, int n) {
@@ -366,6 +366,8 @@ __device__ inline int wrap_or(int g, int n, bool& in) {
     return g;
 }
 
+#include "mgtile.hpp"
+
 // One red-black Gauss-Seidel sweep of TX x TY columns of rows spanning all
 // of z. LDS holds the (TX+4) x (TY+4) rows of p of one tile; red is updated
 // on the tile and its 1-row ring, then black on the tile. Lane r < ROWS
@@ -472,20 +474,14 @@ __device__ __forceinline__ void rb_rows_tiles(const T* __restrict__ pin, const T
     fetch(0, first);
     const T inv_p = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
     auto update = [&](const T* row, int r, int gx, int gy, int z, T b) -> T {
-        T s = T(0);
-        if (P) {
-            s += k.w[2] * row[z + 1 < n2 ? z + 1 : 0];
-            s += k.w[2] * row[z > 0 ? z - 1 : n2 - 1];
-        } else {
-            if (z + 1 < n2) s += k.w[2] * row[z + 1];
-            if (z > 0) s += k.w[2] * row[z - 1];
-        }
-        if (P || gy + 1 < d.n1) s += k.w[1] * box[(r + 1) * n2 + z];
-        if (P || gy > 0) s += k.w[1] * box[(r - 1) * n2 + z];
-        if (P || gx + 1 < d.n0) s += k.w[0] * box[(r + BYr) * n2 + z];
-        if (P || gx > 0) s += k.w[0] * box[(r - BYr) * n2 + z];
+        // a missing neighbour adds zero
+        const T zs = (P || z + 1 < n2 ? row[P && z + 1 == n2 ? 0 : z + 1] : T(0)) +
+                     (P || z > 0 ? row[P && z == 0 ? n2 - 1 : z - 1] : T(0));
+        const T ys = (P || gy + 1 < d.n1 ? box[(r + 1) * n2 + z] : T(0)) + (P || gy > 0 ? box[(r - 1) * n2 + z] : T(0));
+        const T xs = (P || gx + 1 < d.n0 ? box[(r + BYr) * n2 + z] : T(0)) +
+                     (P || gx > 0 ? box[(r - BYr) * n2 + z] : T(0));
         const T inv = P ? inv_p : tab[face_class(gx, d.n0) * 9 + face_class(gy, d.n1) * 3 + face_class(z, n2)];
-        return rb_relax(k, row[z], (b + s) * inv);
+        return rb_relax(k, row[z], gs_value<T>(k, b, zs, ys, xs, inv));
     };
     for (int j = 0; j < count; ++j) {
         const int cur = j & 1;
@@ -646,56 +642,11 @@ __global__ void __launch_bounds__(256) restrict_rows_kernel(const T* __restrict_
     restrict_row<T, P>(p, rhs, coarse, d, k, int(blockIdx.x) * 4 + wave);
 }
 
-// fine += trilinear(coarse); one wavefront per fine row.
-template <class T, bool P>
-__device__ __forceinline__ void prolong_row(const T* __restrict__ coarse, T* __restrict__ fine,
-                                            const Dim32 d, int row) {
-    const int lane = threadIdx.x & 63;
-    if (row >= d.n0 * d.n1) return;
-    const int x = row / d.n1, y = row - x * d.n1;
-    const int C0 = d.n0 / 2, C1 = d.n1 / 2, C2 = d.n2 / 2;
-    const int ax = x / 2 - 1 + (x & 1), ay = y / 2 - 1 + (y & 1);
-    int x0, x1, y0, y1;
-    if (P) {  // -1 <= ax and ax + 1 <= C0
-        x0 = ax < 0 ? ax + C0 : ax; x1 = ax + 1 >= C0 ? ax + 1 - C0 : ax + 1;
-        y0 = ay < 0 ? ay + C1 : ay; y1 = ay + 1 >= C1 ? ay + 1 - C1 : ay + 1;
-    } else {
-        x0 = ax > 0 ? ax : 0; x1 = ax + 1 < C0 - 1 ? ax + 1 : C0 - 1;
-        y0 = ay > 0 ? ay : 0; y1 = ay + 1 < C1 - 1 ? ay + 1 : C1 - 1;
-    }
-    const T wx = (x & 1) ? T(0.25) : T(0.75);
-    const T wy = (y & 1) ? T(0.25) : T(0.75);
-    const T* c00 = coarse + (x0 * C1 + y0) * C2;
-    const T* c01 = coarse + (x0 * C1 + y1) * C2;
-    const T* c10 = coarse + (x1 * C1 + y0) * C2;
-    const T* c11 = coarse + (x1 * C1 + y1) * C2;
-    T* f = fine + (x * d.n1 + y) * d.n2;
-    for (int z = lane; z < d.n2; z += 64) {
-        const int az = z / 2 - 1 + (z & 1);
-        int z0, z1;
-        if (P) { z0 = az < 0 ? az + C2 : az; z1 = az + 1 >= C2 ? az + 1 - C2 : az + 1; }
-        else { z0 = az > 0 ? az : 0; z1 = az + 1 < C2 - 1 ? az + 1 : C2 - 1; }
-        const T wz = (z & 1) ? T(0.25) : T(0.75);
-        const T v00 = c00[z0] * (T(1) - wz) + c00[z1] * wz;
-        const T v01 = c01[z0] * (T(1) - wz) + c01[z1] * wz;
-        const T v10 = c10[z0] * (T(1) - wz) + c10[z1] * wz;
-        const T v11 = c11[z0] * (T(1) - wz) + c11[z1] * wz;
-        f[z] = f[z] + ((v00 * (T(1) - wy) + v01 * wy) * (T(1) - wx) + (v10 * (T(1) - wy) + v11 * wy) * wx);
-    }
-}
-
-template <class T, bool P>
-__global__ void __launch_bounds__(256) prolong_rows_kernel(const T* __restrict__ coarse,
-                                                           T* __restrict__ fine, Dim32 d) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
-    prolong_row<T, P>(coarse, fine, d, int(blockIdx.x) * 4 + wave);
-}
-
-// The same prolongation for a 2x2 group of fine rows: fine rows 2k+1 and
+// fine += trilinear(coarse) for a 2x2 group of fine rows: fine rows 2k+1 and
 // 2k+2 of an axis interpolate between the same coarse rows k and k+1 (only
 // their weights differ), so one wave reads the four coarse rows once and
 // updates up to four fine rows. Group (kx, ky), kx in [-1, C0), ky in
-// [-1, C1); each fine value is formed exactly as prolong_row forms it.
+// [-1, C1).
 template <class T, bool P>
 __global__ void __launch_bounds__(256) prolong_groups_kernel(const T* __restrict__ coarse,
                                                              T* __restrict__ fine, Dim32 d) {
@@ -766,360 +717,6 @@ __global__ void __launch_bounds__(256) prolong_groups_kernel(const T* __restrict
             }
         }
     }
-}
-
-// ---------------------------------------------------------------------------
-// Fused small levels. On levels of up to 64^3 cells a launch costs a few
-// microseconds whatever its size (global-memory round trips and launch
-// gaps, not bytes), so the 2 nu + 2 launches a level takes per V-cycle
-// (nu sweeps, restriction, prolongation, nu sweeps) dominate its time.
-// Two kernels do a level's work in two launches, for nu = 2:
-// * vdown_kernel: the pre-smoothing sweeps, the residual and its
-//   restriction. A workgroup stages its TX x TY tile of full z rows in LDS
-//   with a halo of 2 nu + 1 rows of p and 2 nu rows of rhs, then runs the
-//   2 nu half-sweeps (red, black, red, black) on shrinking regions:
-//   half-sweep s updates the tile and a ring of 2 nu - s rows, whose
-//   neighbours were all updated by half-sweep s - 1. After the last one the
-//   tile and its 1-row ring hold exactly what nu global sweeps produce, so
-//   the residual of the tile and its 2x2x2 averages follow from LDS. The
-//   workgroup writes its tile of p and the coarse cells under the tile.
-// * vup_kernel: the prolongation of the coarse correction and the
-//   post-smoothing sweeps. The coarse rows under the tile and a 2 nu halo
-//   are z-interpolated once each into LDS (the v terms of
-//   prolong_groups_kernel), p + P(e) is formed on the tile and its 2 nu halo
-//   (p read from the pre-smoothed buffer), then 2 nu half-sweeps shrink to
-//   the tile, which is written to the output buffer.
-// Every tile recomputes the halo rows it needs. Each value is formed by the
-// same expressions in the same order as in rb_rows_tiles, restrict_row and
-// prolong_groups_kernel (sweep update, difference-form residual, trilinear
-// weights), so the fused levels reproduce the unfused ones.
-
-constexpr int FUSE_NU = 2;
-constexpr int FUSE_NT = 512;  // threads per fused workgroup
-
-// Box row (bx, by) of a box with halo H around the tile at (x0, y0): the
-// global row (wrapped on periodic axes); false where it lies outside a
-// closed domain. The halo never exceeds an axis extent (checked on the
-// host), so one wrap suffices.
-template <bool P, int H>
-__device__ __forceinline__ bool box_row(int x0, int y0, int bx, int by, const Dim32& d, int& gx, int& gy) {
-    gx = x0 - H + bx;
-    gy = y0 - H + by;
-    if (P) {
-        gx = gx < 0 ? gx + d.n0 : (gx >= d.n0 ? gx - d.n0 : gx);
-        gy = gy < 0 ? gy + d.n1 : (gy >= d.n1 ? gy - d.n1 : gy);
-        return true;
-    }
-    return gx >= 0 && gx < d.n0 && gy >= 0 && gy < d.n1;
-}
-
-// Red-black half-sweep `colour` (0 red: gx + gy + z even) over the tile and
-// a ring of W rows, in place in the p box (BY rows per box x, N2 per row);
-// the rhs box has a halo of H - 1. Same update as rb_rows_tiles. A thread
-// takes its cells in groups of FUSE_ILP: all LDS reads of a group are
-// issued before any of its writes (cells of one colour never read each
-// other), so their latencies overlap.
-constexpr int FUSE_ILP = 4;
-
-template <class T, bool P, int TX, int TY, int N2, int H, int W>
-__device__ __forceinline__ void fused_half_sweep(T* box, const T* rbx, int colour, int x0, int y0,
-                                                 const Dim32& d, const W3<T>& k, const T* tab, T inv_p) {
-    constexpr int BY = TY + 2 * H, RY = BY - 2, H2 = N2 / 2;
-    constexpr int RWY = TY + 2 * W, ITEMS = (TX + 2 * W) * RWY * H2;
-    constexpr int PER = (ITEMS + FUSE_NT - 1) / FUSE_NT;
-#pragma unroll
-    for (int g0 = 0; g0 < PER; g0 += FUSE_ILP) {
-        T val[FUSE_ILP];
-        int at[FUSE_ILP];
-#pragma unroll
-        for (int g = 0; g < FUSE_ILP; ++g) {
-            at[g] = -1;
-            const int i = int(threadIdx.x) + FUSE_NT * (g0 + g);
-            if (g0 + g >= PER || i >= ITEMS) continue;
-            const int rr = i / H2, zl = i % H2;
-            const int bx = H - W + rr / RWY, by = H - W + rr % RWY;
-            int gx, gy;
-            if (!box_row<P, H>(x0, y0, bx, by, d, gx, gy)) continue;
-            const int r = bx * BY + by;
-            const int z = 2 * zl + ((gx + gy + colour) & 1);
-            const T* row = box + r * N2;
-            const T b = rbx[((bx - 1) * RY + (by - 1)) * N2 + z];
-            T s = T(0);
-            if (P) {
-                s += k.w[2] * row[z + 1 < N2 ? z + 1 : 0];
-                s += k.w[2] * row[z > 0 ? z - 1 : N2 - 1];
-            } else {
-                if (z + 1 < N2) s += k.w[2] * row[z + 1];
-                if (z > 0) s += k.w[2] * row[z - 1];
-            }
-            if (P || gy + 1 < d.n1) s += k.w[1] * box[(r + 1) * N2 + z];
-            if (P || gy > 0) s += k.w[1] * box[(r - 1) * N2 + z];
-            if (P || gx + 1 < d.n0) s += k.w[0] * box[(r + BY) * N2 + z];
-            if (P || gx > 0) s += k.w[0] * box[(r - BY) * N2 + z];
-            const T inv = P ? inv_p : tab[face_class(gx, d.n0) * 9 + face_class(gy, d.n1) * 3 + face_class(z, N2)];
-            val[g] = rb_relax(k, row[z], (b + s) * inv);
-            at[g] = r * N2 + z;
-        }
-#pragma unroll
-        for (int g = 0; g < FUSE_ILP; ++g)
-            if (at[g] >= 0) box[at[g]] = val[g];
-    }
-}
-
-// The 2 nu half-sweeps of one smoothing stage; the first updates a ring of
-// W0 rows, each later one a ring one row narrower.
-template <class T, bool P, int TX, int TY, int N2, int H, int W0>
-__device__ __forceinline__ void fused_sweeps(T* box, const T* rbx, int x0, int y0, const Dim32& d,
-                                             const W3<T>& k, const T* tab, T inv_p) {
-    static_assert(2 * FUSE_NU == 4, "four half-sweeps");
-    fused_half_sweep<T, P, TX, TY, N2, H, W0>(box, rbx, 0, x0, y0, d, k, tab, inv_p);
-    __syncthreads();
-    fused_half_sweep<T, P, TX, TY, N2, H, W0 - 1>(box, rbx, 1, x0, y0, d, k, tab, inv_p);
-    __syncthreads();
-    fused_half_sweep<T, P, TX, TY, N2, H, W0 - 2>(box, rbx, 0, x0, y0, d, k, tab, inv_p);
-    __syncthreads();
-    fused_half_sweep<T, P, TX, TY, N2, H, W0 - 3>(box, rbx, 1, x0, y0, d, k, tab, inv_p);
-    __syncthreads();
-}
-
-// Global rows of the p box (halo H) and of the rhs box (halo H - 1) into
-// registers, 16 bytes per load; rows outside a closed domain read as 0.
-template <class T, bool P, int TX, int TY, int N2, int H, int NL, bool RHS>
-__device__ __forceinline__ void fused_fetch(const T* __restrict__ src, uint4 (&v)[NL], int x0, int y0,
-                                            const Dim32& d) {
-    constexpr int CPR = N2 * int(sizeof(T)) / 16;
-    constexpr int BY = TY + 2 * H;
-    constexpr int OX = RHS ? TX + 2 * H - 2 : TX + 2 * H, OY = RHS ? BY - 2 : BY;
-    constexpr int CHUNKS = OX * OY * CPR;
-    static_assert(NL * FUSE_NT >= CHUNKS, "register staging too small");
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int c = int(threadIdx.x) + FUSE_NT * i;
-        v[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (c < CHUNKS) {
-            const int row = c / CPR, part = c % CPR;
-            const int bx = row / OY + (RHS ? 1 : 0), by = row % OY + (RHS ? 1 : 0);
-            int gx, gy;
-            if (box_row<P, H>(x0, y0, bx, by, d, gx, gy))
-                v[i] = reinterpret_cast<const uint4*>(src + (int64_t(gx) * d.n1 + gy) * N2)[part];
-        }
-    }
-}
-
-template <class T, int NL, int CHUNKS>
-__device__ __forceinline__ void fused_store(T* lds, const uint4 (&v)[NL]) {
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int c = int(threadIdx.x) + FUSE_NT * i;
-        if (c < CHUNKS) reinterpret_cast<uint4*>(lds)[c] = v[i];
-    }
-}
-
-// Tile rows of the box to the output level (16-byte stores).
-template <class T, int TX, int TY, int N2, int H>
-__device__ __forceinline__ void fused_write_tile(const T* box, T* __restrict__ out, int x0, int y0,
-                                                 const Dim32& d) {
-    constexpr int CPR = N2 * int(sizeof(T)) / 16, BY = TY + 2 * H;
-    for (int c = threadIdx.x; c < TX * TY * CPR; c += FUSE_NT) {
-        const int row = c / CPR, part = c % CPR;
-        const int lx = row / TY, ly = row % TY;
-        reinterpret_cast<uint4*>(out + (int64_t(x0 + lx) * d.n1 + (y0 + ly)) * N2)[part] =
-            reinterpret_cast<const uint4*>(box + ((H + lx) * BY + (H + ly)) * N2)[part];
-    }
-}
-
-template <class T, bool P, int TX, int TY, int N2>
-struct FusedDown {
-    static constexpr int H = 2 * FUSE_NU + 1;
-    static constexpr int BX = TX + 2 * H, BY = TY + 2 * H, RX = BX - 2, RY = BY - 2;
-    static constexpr int CPR = N2 * int(sizeof(T)) / 16;
-    static constexpr int PCH = BX * BY * CPR, RCH = RX * RY * CPR;
-    static constexpr int NP = (PCH + FUSE_NT - 1) / FUSE_NT, NR = (RCH + FUSE_NT - 1) / FUSE_NT;
-    static constexpr size_t LDS = size_t(BX * BY + RX * RY) * N2 * sizeof(T);
-};
-
-template <class T, bool P, int TX, int TY, int N2>
-struct FusedUp {
-    static constexpr int H = 2 * FUSE_NU;
-    static constexpr int BX = TX + 2 * H, BY = TY + 2 * H, RX = BX - 2, RY = BY - 2;
-    static constexpr int CX = TX / 2 + H + 2, CY = TY / 2 + H + 2, C2 = N2 / 2;
-    static constexpr int CPR = N2 * int(sizeof(T)) / 16, CCPR = C2 * int(sizeof(T)) / 16;
-    static constexpr int PCH = BX * BY * CPR, RCH = RX * RY * CPR, CCH = CX * CY * CCPR;
-    static constexpr int NP = (PCH + FUSE_NT - 1) / FUSE_NT, NR = (RCH + FUSE_NT - 1) / FUSE_NT, NC = (CCH + FUSE_NT - 1) / FUSE_NT;
-    static constexpr size_t LDS = size_t(BX * BY + RX * RY) * N2 * sizeof(T) +
-                                  size_t(CX * CY) * (C2 + N2) * sizeof(T);
-};
-
-// nu = 2 pre-smoothing sweeps of pin (zero_in: of a zero iterate) into the
-// tile of pout, and coarse = avg8(rhs - A p) under the tile.
-template <class T, bool P, int TX, int TY, int N2>
-__global__ void __launch_bounds__(FUSE_NT) vdown_kernel(const T* __restrict__ pin, const T* __restrict__ rhs,
-                                                    T* __restrict__ pout, T* __restrict__ coarse, Dim32 d,
-                                                    W3<T> k, int zero_in, int ntx, int nty) {
-    using G = FusedDown<T, P, TX, TY, N2>;
-    constexpr int H = G::H, BY = G::BY, RY = G::RY, C2 = N2 / 2;
-    static_assert(TX % 2 == 0 && TY % 2 == 0 && N2 % 32 == 0 && N2 <= 128, "fused tile shape");
-    extern __shared__ unsigned char raw[];
-    T* box = reinterpret_cast<T*>(raw);
-    T* rbx = box + G::BX * BY * N2;
-    __shared__ T tab[27];
-    const int tile = int(xcd_tile(blockIdx.x, int64_t(ntx) * nty));
-    const int x0 = (tile / nty) * TX, y0 = (tile % nty) * TY;
-    {
-        uint4 vp[G::NP], vr[G::NR];
-        if (zero_in) {
-#pragma unroll
-            for (int i = 0; i < G::NP; ++i) vp[i] = make_uint4(0u, 0u, 0u, 0u);
-        } else {
-            fused_fetch<T, P, TX, TY, N2, H, G::NP, false>(pin, vp, x0, y0, d);
-        }
-        fused_fetch<T, P, TX, TY, N2, H, G::NR, true>(rhs, vr, x0, y0, d);
-        fused_store<T, G::NP, G::PCH>(box, vp);
-        fused_store<T, G::NR, G::RCH>(rbx, vr);
-    }
-    if (!P && threadIdx.x < 27) tab[threadIdx.x] = inv_diag_entry<T>(threadIdx.x, k);
-    __syncthreads();
-    const T inv_p = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
-    fused_sweeps<T, P, TX, TY, N2, H, H - 1>(box, rbx, x0, y0, d, k, tab, inv_p);
-    fused_write_tile<T, TX, TY, N2, H>(box, pout, x0, y0, d);
-    // residual on the tile (difference form of apply_row) and its 2x2x2
-    // averages, summed in restrict_row's order
-    const int C1 = d.n1 / 2;
-    for (int i = threadIdx.x; i < (TX / 2) * (TY / 2) * C2; i += FUSE_NT) {
-        const int cr = i / C2, cz = i % C2;
-        const int cxl = cr / (TY / 2), cyl = cr % (TY / 2);
-        T v = T(0);
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int lx = 2 * cxl + a, ly = 2 * cyl + b;
-                const int gx = x0 + lx, gy = y0 + ly;
-                const int r = (H + lx) * BY + (H + ly);
-                const T* row = box + r * N2;
-                const T* rr = rbx + ((H - 1 + lx) * RY + (H - 1 + ly)) * N2;
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const int z = 2 * cz + c;
-                    const T cv = row[z];
-                    T ap = T(0);
-                    if (P) {
-                        ap += k.w[0] * (cv - box[(r + BY) * N2 + z]);
-                        ap += k.w[0] * (cv - box[(r - BY) * N2 + z]);
-                        ap += k.w[1] * (cv - box[(r + 1) * N2 + z]);
-                        ap += k.w[1] * (cv - box[(r - 1) * N2 + z]);
-                        ap += k.w[2] * (cv - row[z + 1 < N2 ? z + 1 : 0]);
-                        ap += k.w[2] * (cv - row[z > 0 ? z - 1 : N2 - 1]);
-                    } else {
-                        if (gx + 1 < d.n0) ap += k.w[0] * (cv - box[(r + BY) * N2 + z]);
-                        if (gx > 0) ap += k.w[0] * (cv - box[(r - BY) * N2 + z]);
-                        if (gy + 1 < d.n1) ap += k.w[1] * (cv - box[(r + 1) * N2 + z]);
-                        if (gy > 0) ap += k.w[1] * (cv - box[(r - 1) * N2 + z]);
-                        if (z + 1 < N2) ap += k.w[2] * (cv - row[z + 1]);
-                        if (z > 0) ap += k.w[2] * (cv - row[z - 1]);
-                    }
-                    v += rr[z] - ap;
-                }
-            }
-        coarse[(int64_t(x0 / 2 + cxl) * C1 + (y0 / 2 + cyl)) * C2 + cz] = v * T(0.125);
-    }
-}
-
-// pout = nu = 2 post-smoothing sweeps of pin + trilinear(coarse), tile by
-// tile.
-template <class T, bool P, int TX, int TY, int N2>
-__global__ void __launch_bounds__(FUSE_NT) vup_kernel(const T* __restrict__ pin, const T* __restrict__ coarse,
-                                                  const T* __restrict__ rhs, T* __restrict__ pout, Dim32 d,
-                                                  W3<T> k, int ntx, int nty) {
-    using G = FusedUp<T, P, TX, TY, N2>;
-    constexpr int H = G::H, BY = G::BY, CX = G::CX, CY = G::CY, C2 = G::C2;
-    static_assert(TX % 2 == 0 && TY % 2 == 0 && N2 % 32 == 0 && N2 <= 128, "fused tile shape");
-    extern __shared__ unsigned char raw[];
-    T* box = reinterpret_cast<T*>(raw);
-    T* rbx = box + G::BX * BY * N2;
-    T* craw = rbx + G::RX * G::RY * N2;  // CX*CY coarse rows of C2
-    T* vz = craw + CX * CY * C2;         // the same rows z-interpolated to N2
-    __shared__ T tab[27];
-    const int tile = int(xcd_tile(blockIdx.x, int64_t(ntx) * nty));
-    const int x0 = (tile / nty) * TX, y0 = (tile % nty) * TY;
-    const int C0 = d.n0 / 2, C1 = d.n1 / 2;
-    // coarse row ia of the staged block is the unwrapped coarse x index
-    // ax_lo + ia (wrapped, or clamped on a closed axis as prolong_groups
-    // clamps it)
-    const int ax_lo = x0 / 2 - FUSE_NU - 1, ay_lo = y0 / 2 - FUSE_NU - 1;
-    uint4 vp[G::NP], vr[G::NR];
-    fused_fetch<T, P, TX, TY, N2, H, G::NP, false>(pin, vp, x0, y0, d);
-    fused_fetch<T, P, TX, TY, N2, H, G::NR, true>(rhs, vr, x0, y0, d);
-    {
-        uint4 vc[G::NC];
-#pragma unroll
-        for (int i = 0; i < G::NC; ++i) {
-            const int c = int(threadIdx.x) + FUSE_NT * i;
-            vc[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (c < G::CCH) {
-                const int row = c / G::CCPR, part = c % G::CCPR;
-                int cx = ax_lo + row / CY, cy = ay_lo + row % CY;
-                if (P) {
-                    cx = cx < 0 ? cx + C0 : (cx >= C0 ? cx - C0 : cx);
-                    cy = cy < 0 ? cy + C1 : (cy >= C1 ? cy - C1 : cy);
-                } else {
-                    cx = cx < 0 ? 0 : (cx > C0 - 1 ? C0 - 1 : cx);
-                    cy = cy < 0 ? 0 : (cy > C1 - 1 ? C1 - 1 : cy);
-                }
-                vc[i] = reinterpret_cast<const uint4*>(coarse + (int64_t(cx) * C1 + cy) * C2)[part];
-            }
-        }
-        fused_store<T, G::NC, G::CCH>(craw, vc);
-    }
-    if (!P && threadIdx.x < 27) tab[threadIdx.x] = inv_diag_entry<T>(threadIdx.x, k);
-    __syncthreads();
-    for (int i = threadIdx.x; i < CX * CY * N2; i += FUSE_NT) {
-        const int row = i / N2, z = i % N2;
-        const int az = z / 2 - 1 + (z & 1);
-        int z0, z1;
-        if (P) { z0 = az < 0 ? az + C2 : az; z1 = az + 1 >= C2 ? az + 1 - C2 : az + 1; }
-        else { z0 = az > 0 ? az : 0; z1 = az + 1 < C2 - 1 ? az + 1 : C2 - 1; }
-        const T wz = (z & 1) ? T(0.25) : T(0.75);
-        const T* c = craw + row * C2;
-        vz[i] = c[z0] * (T(1) - wz) + c[z1] * wz;
-    }
-    fused_store<T, G::NR, G::RCH>(rbx, vr);
-    __syncthreads();
-    // p + P(e) on the box (rows outside a closed domain stay unused)
-    constexpr int VEC = 16 / int(sizeof(T));
-#pragma unroll
-    for (int i = 0; i < G::NP; ++i) {
-        const int c = int(threadIdx.x) + FUSE_NT * i;
-        if (c >= G::PCH) continue;
-        const int row = c / G::CPR, part = c % G::CPR;
-        const int bx = row / BY, by = row % BY;
-        int gx, gy;
-        union { uint4 u; T t[VEC]; } val;
-        val.u = vp[i];
-        if (box_row<P, H>(x0, y0, bx, by, d, gx, gy)) {  // reads only: vz and registers
-            const int ux = x0 - H + bx, uy = y0 - H + by;  // unwrapped fine row
-            const int ia = ((ux - 1) >> 1) - ax_lo, ib = ((uy - 1) >> 1) - ay_lo;
-            const T* v00 = vz + (ia * CY + ib) * N2;
-            const T* v01 = vz + (ia * CY + ib + 1) * N2;
-            const T* v10 = vz + ((ia + 1) * CY + ib) * N2;
-            const T* v11 = vz + ((ia + 1) * CY + ib + 1) * N2;
-            const T wx = (ux & 1) ? T(0.25) : T(0.75);
-            const T wy = (uy & 1) ? T(0.25) : T(0.75);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                const int z = part * VEC + e;
-                val.t[e] = val.t[e] + ((v00[z] * (T(1) - wy) + v01[z] * wy) * (T(1) - wx) +
-                                       (v10[z] * (T(1) - wy) + v11[z] * wy) * wx);
-            }
-        }
-        vp[i] = val.u;
-    }
-    // all vz reads above are issued before the box writes below
-    fused_store<T, G::NP, G::PCH>(box, vp);
-    __syncthreads();
-    const T inv_p = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
-    fused_sweeps<T, P, TX, TY, N2, H, H - 1>(box, rbx, x0, y0, d, k, tab, inv_p);
-    fused_write_tile<T, TX, TY, N2, H>(box, pout, x0, y0, d);
 }
 
 // per-workgroup [sum r, sum r^2, sum |r|, non-finite] of r = rhs - A p,
@@ -1570,27 +1167,9 @@ __device__ inline int find_entry(const D* __restrict__ desc, int n, int b) {
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
-template <class T>
-struct SweepDesc {
-    const T* pin;
-    const T* rhs;
-    T* pout;
+struct StageDesc {
+    StageArgs<float> a;
     const int32_t* active;
-    Dim32 d;
-    W3<T> k;
-    int ntx, nty;
-    int begin;
-    int zero_in;
-};
-
-template <class T>
-struct RowDesc {
-    const T* a;  // restriction: p; prolongation: coarse p
-    const T* b;  // restriction: rhs
-    T* c;        // restriction: coarse rhs; prolongation: fine p
-    const int32_t* active;
-    Dim32 d;     // fine level
-    W3<T> k;
     int begin;
 };
 
@@ -1614,34 +1193,14 @@ struct VecDesc {
 
 constexpr int VEC_CHUNK = 4096;  // elements per workgroup in batched vector passes
 
-template <class T, bool P>
-__global__ void __launch_bounds__(256) rb_rows_batch_kernel(const SweepDesc<T>* __restrict__ desc,
-                                                            int n) {
+template <bool P, int TX, int NPH, bool RESTRICT>
+__global__ void __launch_bounds__((Tile3<float, TX, 8, NPH, RESTRICT>::NT)) stage_batch_kernel(
+    const StageDesc* __restrict__ desc, int n) {
+    extern __shared__ unsigned char raw[];
     const int b = blockIdx.x;
-    const SweepDesc<T>& s = desc[find_entry(desc, n, b)];
-    if (s.active && s.active[0] == 0) return;  // uniform over the workgroup
-    rb_rows_tiles<T, P, 2, 2, 0>(s.pin, s.rhs, s.pout, s.d, s.k, s.zero_in, s.ntx, s.nty,
-                                 b - s.begin, 1, 1);
-}
-
-template <class T, bool P>
-__global__ void __launch_bounds__(256) restrict_batch_kernel(const RowDesc<T>* __restrict__ desc,
-                                                             int n) {
-    const int b = blockIdx.x;
-    const RowDesc<T>& s = desc[find_entry(desc, n, b)];
-    if (s.active && s.active[0] == 0) return;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    restrict_row<T, P>(s.a, s.b, s.c, s.d, s.k, (b - s.begin) * 4 + wave);
-}
-
-template <class T, bool P>
-__global__ void __launch_bounds__(256) prolong_batch_kernel(const RowDesc<T>* __restrict__ desc,
-                                                            int n) {
-    const int b = blockIdx.x;
-    const RowDesc<T>& s = desc[find_entry(desc, n, b)];
-    if (s.active && s.active[0] == 0) return;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    prolong_row<T, P>(s.a, s.c, s.d, (b - s.begin) * 4 + wave);
+    const StageDesc& s = desc[find_entry(desc, n, b)];
+    if (s.active[0] == 0) return;  // uniform over the workgroup
+    stage_tile<float, P, true, TX, 8, NPH, RESTRICT>(s.a, b - s.begin, reinterpret_cast<float*>(raw));
 }
 
 template <class T, bool P>
@@ -1963,81 +1522,85 @@ struct FastRunner {
         return OK;
     }
 
-    // Tile of the fused down/up launches at level l: 2 for 2x2, 4 for 4x4
-    // (FP32) or 4x2 (FP64) rows; 0 where the level runs unfused.
-    int fuse_code(int l) const {
-        if (pl.smoother != 1 || pl.nu != FUSE_NU || l >= coarse_first || pl.fuse_cells < 0) return 0;
-        const int64_t limit = pl.fuse_cells > 0 ? int64_t(pl.fuse_cells) : (int64_t(1) << 18);
-        const int64_t n0 = pl.n[l][0], n1 = pl.n[l][1], n2 = pl.n[l][2];
-        if (cells(l) > limit || (n2 != 32 && n2 != 64)) return 0;
-        const int code = n2 == 64 ? 4 : 2;
-        const int tx = code, ty = (code == 4 && sizeof(T) == 8) ? 2 : code;
-        if (n0 % tx || n1 % ty || n0 < 2 * FUSE_NU + 1 || n1 < 2 * FUSE_NU + 1) return 0;
+    // Whether level l's smoothing stages run as stage launches.
+    bool staged(int l) const {
+        if (pl.n[l][1] * pl.n[l][2] >= (int64_t(1) << 28)) return false;  // 32-bit byte offsets in a plane
+        if (l >= coarse_first || pl.fuse_cells < 0 || (pl.fuse_cells > 0 && cells(l) > int64_t(pl.fuse_cells))) return false;
         const void* ptrs[4] = {pl.p[l], pl.tmp[l], pl.rhs[l], pl.p[l + 1]};
         for (const void* q : ptrs)
-            if (reinterpret_cast<uintptr_t>(q) % 16) return 0;
-        return code;
+            if (reinterpret_cast<uintptr_t>(q) % 16) return false;
+        return true;
     }
 
-    template <int TX, int TY, int N2>
-    int vdown_n(int l, const T* in, T* out, bool zero_in) const {
-        const Dim32 d = D(l);
-        const int ntx = d.n0 / TX, nty = d.n1 / TY;
-        const size_t bytes = FusedDown<T, true, TX, TY, N2>::LDS;
-        const void* fn = pl.periodic ? reinterpret_cast<const void*>(vdown_kernel<T, true, TX, TY, N2>)
-                                     : reinterpret_cast<const void*>(vdown_kernel<T, false, TX, TY, N2>);
-        if (int r = dynamic_lds(fn, bytes)) return r;
-        const unsigned g = unsigned(ntx * nty);
-        if (pl.periodic)
-            vdown_kernel<T, true, TX, TY, N2><<<g, FUSE_NT, bytes, s>>>(in, R(l), out, R(l + 1), d, K(l), zero_in, ntx, nty);
-        else
-            vdown_kernel<T, false, TX, TY, N2><<<g, FUSE_NT, bytes, s>>>(in, R(l), out, R(l + 1), d, K(l), zero_in, ntx, nty);
+    template <bool Per, bool GS, int TX, int TY, int NPH, bool RESTRICT>
+    int stage_n(const StageArgs<T>& a) const {
+        using G = Tile3<T, TX, TY, NPH, RESTRICT>;
+        if (int r = dynamic_lds(reinterpret_cast<const void*>(stage_kernel<T, Per, GS, TX, TY, NPH, RESTRICT>), G::LDS)) return r;
+        const int tiles = stage_tiles(a.d, TX, TY);
+        stage_kernel<T, Per, GS, TX, TY, NPH, RESTRICT><<<unsigned(tiles), G::NT, G::LDS, s>>>(a, tiles);
         AFSI_LAUNCH_CHECK();
         return OK;
     }
 
-    template <int TX, int TY, int N2>
-    int vup_n(int l, const T* in, const T* cc, T* out) const {
-        const Dim32 d = D(l);
-        const int ntx = d.n0 / TX, nty = d.n1 / TY;
-        const size_t bytes = FusedUp<T, true, TX, TY, N2>::LDS;
-        const void* fn = pl.periodic ? reinterpret_cast<const void*>(vup_kernel<T, true, TX, TY, N2>)
-                                     : reinterpret_cast<const void*>(vup_kernel<T, false, TX, TY, N2>);
-        if (int r = dynamic_lds(fn, bytes)) return r;
-        const unsigned g = unsigned(ntx * nty);
-        if (pl.periodic)
-            vup_kernel<T, true, TX, TY, N2><<<g, FUSE_NT, bytes, s>>>(in, cc, R(l), out, d, K(l), ntx, nty);
-        else
-            vup_kernel<T, false, TX, TY, N2><<<g, FUSE_NT, bytes, s>>>(in, cc, R(l), out, d, K(l), ntx, nty);
-        AFSI_LAUNCH_CHECK();
+    template <int TX, int TY, int NPH, bool GS>
+    int stage_tx(const StageArgs<T>& a) const {
+        if (pl.periodic) return a.restricted ? stage_n<true, GS, TX, TY, NPH, true>(a) : stage_n<true, GS, TX, TY, NPH, false>(a);
+        return a.restricted ? stage_n<false, GS, TX, TY, NPH, true>(a) : stage_n<false, GS, TX, TY, NPH, false>(a);
+    }
+
+    // Phases per launch and tile of a level. Two phases keep the halo small
+    // where the level fills the chip several times over (redundant cells are
+    // then the cost); smaller levels are bound by launches and by the length of
+    // one workgroup's instruction stream, so they take four phases and, up to
+    // 256 (down) or below 256 (up) 8x8 tiles, the shorter 4x8 tile. Measured,
+    // periodic red-black, us per V(2,2) level visit (down + up):
+    //   FP32 128^3: 4 x 11-14 (two phases) 46, four phases 55, sweep kernels 56
+    //   FP64 128^3: 70, 89, 106
+    //   FP32 64^3: two phases 21 (and two more launches), 4x8 / 8x8 15
+    //   FP64 64^3: 21, 19; one fused launch per stage on full z rows took 40
+    static constexpr int64_t WIDE_TILES = 1024;
+    bool wide(int l) const { return stage_tiles(D(l), 8, 8) >= WIDE_TILES; }
+
+    template <bool GS>
+    int stage_launch(const StageArgs<T>& a, bool wide_level, bool up) const {
+        if (wide_level) return stage_tx<8, 8, 2, GS>(a);
+        const int tiles = stage_tiles(a.d, 8, 8);
+        return (up ? tiles < 256 : tiles <= 256) ? stage_tx<4, 8, 4, GS>(a) : stage_tx<8, 8, 4, GS>(a);
+    }
+
+    // One smoothing stage of level l (restriction or prolongation included)
+    // as launches of a few phases; p and tmp alternate.
+    int stage(int l, T*& cur, bool up, const T* coarse, bool zero) const {
+        const bool two = wide(l);
+        const int per = two ? 2 : 4;
+        const int phases = pl.smoother == 1 ? 2 * pl.nu : pl.nu, chunks = (phases + per - 1) / per;
+        for (int c = 0; c < chunks; ++c) {
+            StageArgs<T> a{};
+            a.in = cur;
+            a.rhs = R(l);
+            a.out = cur == P(l) ? W(l) : P(l);
+            a.coarse = up && c == 0 ? coarse : nullptr;
+            a.restricted = !up && c == chunks - 1 ? R(l + 1) : nullptr;
+            a.d = D(l);
+            a.k = K(l);
+            a.omega = T(pl.omega);
+            a.first = c * per;
+            a.count = phases - a.first < per ? phases - a.first : per;
+            a.zero = zero && c == 0;
+            const int r = pl.smoother == 1 ? stage_launch<true>(a, two, up) : stage_launch<false>(a, two, up);
+            if (r) return r;
+            cur = a.out;
+        }
         return OK;
-    }
-
-    int vdown(int code, int l, const T* in, T* out, bool zero_in) const {
-        constexpr int TY4 = sizeof(T) == 8 ? 2 : 4;
-        if (code == 2)
-            return D(l).n2 == 64 ? vdown_n<2, 2, 64>(l, in, out, zero_in) : vdown_n<2, 2, 32>(l, in, out, zero_in);
-        return D(l).n2 == 64 ? vdown_n<4, TY4, 64>(l, in, out, zero_in) : vdown_n<4, TY4, 32>(l, in, out, zero_in);
-    }
-
-    int vup(int code, int l, const T* in, const T* cc, T* out) const {
-        constexpr int TY4 = sizeof(T) == 8 ? 2 : 4;
-        if (code == 2) return D(l).n2 == 64 ? vup_n<2, 2, 64>(l, in, cc, out) : vup_n<2, 2, 32>(l, in, cc, out);
-        return D(l).n2 == 64 ? vup_n<4, TY4, 64>(l, in, cc, out) : vup_n<4, TY4, 32>(l, in, cc, out);
     }
 
     int cycle(int l, T*& cur, bool zero_initial = false) const {
         if (l == coarse_first) return coarse(l, (l == 0 && !zero_initial) ? cur : nullptr, cur);
-        if (const int code = fuse_code(l)) {
-            T* out = cur == P(l) ? W(l) : P(l);
-            if (int r = vdown(code, l, cur, out, l > 0 || zero_initial)) return r;
-            cur = out;
+        if (staged(l)) {  // as many launches up as down: the iterate ends in cur's first buffer
+            if (int r = stage(l, cur, false, nullptr, l > 0 || zero_initial)) return r;
             T* cc = P(l + 1);
             if (int r = cycle(l + 1, cc)) return r;
-            out = cur == P(l) ? W(l) : P(l);
-            if (int r = vup(code, l, cur, cc, out)) return r;
-            cur = out;
-            return OK;
+            return stage(l, cur, true, cc, false);
         }
         // coarse iterates (and a zero initial level-0 iterate) start at zero
         if (int r = smooth(l, cur, l > 0 || zero_initial)) return r;
@@ -2159,11 +1722,11 @@ struct BatchLayout {
     int n = 0, levels = 0, nu = 0, periodic = 0;
     int cf[1024];                      // first LDS-solved level per instance
     std::vector<int> members[AFSI_MG_MAX_LEVELS];
-    size_t sweep_off[AFSI_MG_MAX_LEVELS][3];  // k = 0 (zero input), even k, odd k
-    int sweep_blocks[AFSI_MG_MAX_LEVELS];
-    size_t sweep_lds[AFSI_MG_MAX_LEVELS];
-    size_t restrict_off[AFSI_MG_MAX_LEVELS], prolong_off[AFSI_MG_MAX_LEVELS];
-    int restrict_blocks[AFSI_MG_MAX_LEVELS], prolong_blocks[AFSI_MG_MAX_LEVELS];
+    // smoothing stages of a level: `chunks` launches down (desc 0..chunks-1),
+    // as many up, and the first down launch of a later inner cycle (last desc)
+    size_t stage_off[AFSI_MG_MAX_LEVELS];
+    int tile_x[AFSI_MG_MAX_LEVELS], phases[AFSI_MG_MAX_LEVELS], chunks[AFSI_MG_MAX_LEVELS];
+    int stage_blocks[AFSI_MG_MAX_LEVELS];
     size_t coarse_off[2] = {0, 0}, coarse_lds = 0;  // first cycle of an iteration (zero start); later ones
     size_t ref_off[4] = {0, 0, 0, 0};  // residual of x[0]; step from x[0]; step from x[1]; residual of x[1]
     int ref_blocks = 0;
@@ -2199,31 +1762,26 @@ static int batch_layout(const afsi_mgb_batch* bt, BatchLayout& L) {
     int64_t partials = 0;
     for (int l = 0; l < L.levels; ++l) {
         L.members[l].clear();
-        int sb = 0, rb = 0, pb = 0;
-        size_t lds = 0;
+        int64_t tiles = 0;
         for (int i = 0; i < L.n; ++i) {
             if (l >= L.cf[i]) continue;
             L.members[l].push_back(i);
             const int64_t* nn = bt->items[i].plan.n[l];
-            sb += int((nn[0] / 2) * (nn[1] / 2));
-            rb += int(cdiv((nn[0] / 2) * (nn[1] / 2), 4));
-            pb += int(cdiv(nn[0] * nn[1], 4));
-            const size_t box = size_t(6 * 6) * size_t(nn[2]) * sizeof(float);
-            if (box > lds) lds = box;
+            tiles += stage_tiles(Dim32{int(nn[0]), int(nn[1]), int(nn[2])}, 8, 8);
         }
-        L.sweep_blocks[l] = sb;
-        L.restrict_blocks[l] = rb;
-        L.prolong_blocks[l] = pb;
-        L.sweep_lds[l] = lds;
-        const size_t m = L.members[l].size();
-        for (int v = 0; v < 3; ++v) {
-            L.sweep_off[l][v] = off;
-            off = align64(off + m * sizeof(SweepDesc<float>));
+        // the rule of FastRunner::wide and stage_launch over the whole level
+        L.phases[l] = tiles >= FastRunner<float>::WIDE_TILES ? 2 : 4;
+        L.tile_x[l] = tiles < 256 ? 4 : 8;
+        L.chunks[l] = (2 * L.nu + L.phases[l] - 1) / L.phases[l];
+        int64_t blocks = 0;
+        for (int i : L.members[l]) {
+            const int64_t* nn = bt->items[i].plan.n[l];
+            blocks += stage_tiles(Dim32{int(nn[0]), int(nn[1]), int(nn[2])}, L.tile_x[l], 8);
         }
-        L.restrict_off[l] = off;
-        off = align64(off + m * sizeof(RowDesc<float>));
-        L.prolong_off[l] = off;
-        off = align64(off + m * sizeof(RowDesc<float>));
+        AFSI_REQUIRE(blocks < (int64_t(1) << 30), "batch level too large");
+        L.stage_blocks[l] = int(blocks);
+        L.stage_off[l] = off;
+        off = align64(off + L.members[l].size() * size_t(2 * L.chunks[l] + 1) * sizeof(StageDesc));
     }
     for (int c = 0; c < 2; ++c) {
         L.coarse_off[c] = off;
@@ -2271,30 +1829,35 @@ static int batch_prepare(const afsi_mgb_batch* bt, hipStream_t s) {
     std::vector<char> host(L.total, 0);
     void* hw = host.data();
     for (int l = 0; l < L.levels; ++l) {
-        int sb = 0, rb = 0, pb = 0;
-        for (size_t j = 0; j < L.members[l].size(); ++j) {
+        int begin = 0;
+        const size_t m = L.members[l].size();
+        StageDesc* descs = at<StageDesc>(hw, L.stage_off[l]);
+        for (size_t j = 0; j < m; ++j) {
             const int i = L.members[l][j];
             const afsi_mg3d_plan& pl = bt->items[i].plan;
-            const Dim32 d{int(pl.n[l][0]), int(pl.n[l][1]), int(pl.n[l][2])};
-            W3<float> k;
-            for (int a = 0; a < 3; ++a) k.w[a] = float(pl.inv_h2[l][a]);
-            k.relax = float(pl.relax > 0.0 ? pl.relax : 1.0);
-            float* P = static_cast<float*>(pl.p[l]);
-            float* W = static_cast<float*>(pl.tmp[l]);
-            const float* R = static_cast<const float*>(pl.rhs[l]);
-            const int ntx = d.n0 / 2, nty = d.n1 / 2;
-            const int32_t* act = bt->active + i;
-            at<SweepDesc<float>>(hw, L.sweep_off[l][0])[j] = SweepDesc<float>{P, R, W, act, d, k, ntx, nty, sb, 1};
-            at<SweepDesc<float>>(hw, L.sweep_off[l][1])[j] = SweepDesc<float>{P, R, W, act, d, k, ntx, nty, sb, 0};
-            at<SweepDesc<float>>(hw, L.sweep_off[l][2])[j] = SweepDesc<float>{W, R, P, act, d, k, ntx, nty, sb, 0};
-            float* cur = (L.nu % 2) ? W : P;  // iterate after the pre-smoothing sweeps
-            at<RowDesc<float>>(hw, L.restrict_off[l])[j] =
-                RowDesc<float>{cur, R, static_cast<float*>(pl.rhs[l + 1]), act, d, k, rb};
-            at<RowDesc<float>>(hw, L.prolong_off[l])[j] =
-                RowDesc<float>{static_cast<const float*>(pl.p[l + 1]), nullptr, cur, act, d, k, pb};
-            sb += ntx * nty;
-            rb += int(cdiv(int64_t(d.n0 / 2) * (d.n1 / 2), 4));
-            pb += int(cdiv(int64_t(d.n0) * d.n1, 4));
+            float* buffers[2] = {static_cast<float*>(pl.p[l]), static_cast<float*>(pl.tmp[l])};
+            StageArgs<float> a{};
+            a.rhs = static_cast<const float*>(pl.rhs[l]);
+            a.d = Dim32{int(pl.n[l][0]), int(pl.n[l][1]), int(pl.n[l][2])};
+            for (int q = 0; q < 3; ++q) a.k.w[q] = float(pl.inv_h2[l][q]);
+            a.k.relax = float(pl.relax > 0.0 ? pl.relax : 1.0);
+            for (int c = 0; c < 2 * L.chunks[l]; ++c) {
+                const bool up = c >= L.chunks[l];
+                const int k = up ? c - L.chunks[l] : c;
+                a.in = buffers[c & 1];
+                a.out = buffers[1 - (c & 1)];
+                a.coarse = up && k == 0 ? static_cast<const float*>(pl.p[l + 1]) : nullptr;
+                a.restricted = !up && k == L.chunks[l] - 1 ? static_cast<float*>(pl.rhs[l + 1]) : nullptr;
+                a.first = k * L.phases[l];
+                a.count = std::min(L.phases[l], 2 * L.nu - a.first);
+                a.zero = c == 0;  // a cycle starts from zero
+                descs[size_t(c) * m + j] = StageDesc{a, bt->active + i, begin};
+                if (c == 0) {  // except on level 0 of a later cycle of one refinement iteration
+                    a.zero = 0;
+                    descs[size_t(2 * L.chunks[l]) * m + j] = StageDesc{a, bt->active + i, begin};
+                }
+            }
+            begin += stage_tiles(a.d, L.tile_x[l], 8);
         }
     }
     int rbeg = 0, vbeg = 0;
@@ -2352,41 +1915,42 @@ static int batch_prepare(const afsi_mgb_batch* bt, hipStream_t s) {
     return OK;
 }
 
+template <bool P, int TX, int NPH, bool RESTRICT>
+static int batch_stage_n(const StageDesc* desc, int m, int blocks, hipStream_t s) {
+    using G = Tile3<float, TX, 8, NPH, RESTRICT>;
+    if (int r = dynamic_lds(reinterpret_cast<const void*>(stage_batch_kernel<P, TX, NPH, RESTRICT>), G::LDS)) return r;
+    stage_batch_kernel<P, TX, NPH, RESTRICT><<<unsigned(blocks), G::NT, G::LDS, s>>>(desc, m);
+    AFSI_LAUNCH_CHECK();
+    return OK;
+}
+
+template <bool P>
+static int batch_stage(const BatchLayout& L, int l, const StageDesc* desc, bool restricts, hipStream_t s) {
+    const int m = int(L.members[l].size()), blocks = L.stage_blocks[l];
+    if (L.phases[l] == 2)
+        return restricts ? batch_stage_n<P, 8, 2, true>(desc, m, blocks, s) : batch_stage_n<P, 8, 2, false>(desc, m, blocks, s);
+    if (L.tile_x[l] == 4)
+        return restricts ? batch_stage_n<P, 4, 4, true>(desc, m, blocks, s) : batch_stage_n<P, 4, 4, false>(desc, m, blocks, s);
+    return restricts ? batch_stage_n<P, 8, 4, true>(desc, m, blocks, s) : batch_stage_n<P, 8, 4, false>(desc, m, blocks, s);
+}
+
 template <bool P>
 static int batch_vcycle(const afsi_mgb_batch* bt, const BatchLayout& L, hipStream_t s, bool first = true) {
     void* ws = bt->workspace;
-    const void* sweep_fn = reinterpret_cast<const void*>(rb_rows_batch_kernel<float, P>);
-    for (int l = 0; l < L.levels; ++l) {
-        const int m = int(L.members[l].size());
-        if (int r = dynamic_lds(sweep_fn, L.sweep_lds[l])) return r;
-        for (int it = 0; it < L.nu; ++it) {
-            // the first sweep of a cycle starts from zero, except on level 0
-            // of a later cycle of one refinement iteration (which continues
-            // from the correction so far)
-            const int v = it == 0 ? (l == 0 && !first ? 1 : 0) : (it % 2 ? 2 : 1);
-            rb_rows_batch_kernel<float, P><<<unsigned(L.sweep_blocks[l]), 256, L.sweep_lds[l], s>>>(
-                at<SweepDesc<float>>(ws, L.sweep_off[l][v]), m);
+    const auto desc = [&](int l, int c) { return at<StageDesc>(ws, L.stage_off[l]) + size_t(c) * L.members[l].size(); };
+    for (int l = 0; l < L.levels; ++l)
+        for (int c = 0; c < L.chunks[l]; ++c) {
+            const bool later = c == 0 && l == 0 && !first;
+            if (int r = batch_stage<P>(L, l, desc(l, later ? 2 * L.chunks[l] : c), c == L.chunks[l] - 1, s)) return r;
         }
-        restrict_batch_kernel<float, P><<<unsigned(L.restrict_blocks[l]), 256, 0, s>>>(
-            at<RowDesc<float>>(ws, L.restrict_off[l]), m);
-        AFSI_LAUNCH_CHECK();
-    }
     const void* coarse_fn = reinterpret_cast<const void*>(coarse_batch_kernel<float, P>);
     if (int r = dynamic_lds(coarse_fn, L.coarse_lds)) return r;
     coarse_batch_kernel<float, P><<<unsigned(L.n), COARSE_THREADS, L.coarse_lds, s>>>(
         at<CoarseArgs<float>>(ws, L.coarse_off[first ? 0 : 1]));
     AFSI_LAUNCH_CHECK();
-    for (int l = L.levels - 1; l >= 0; --l) {
-        const int m = int(L.members[l].size());
-        prolong_batch_kernel<float, P><<<unsigned(L.prolong_blocks[l]), 256, 0, s>>>(
-            at<RowDesc<float>>(ws, L.prolong_off[l]), m);
-        for (int it = L.nu; it < 2 * L.nu; ++it) {
-            const int v = it % 2 ? 2 : 1;
-            rb_rows_batch_kernel<float, P><<<unsigned(L.sweep_blocks[l]), 256, L.sweep_lds[l], s>>>(
-                at<SweepDesc<float>>(ws, L.sweep_off[l][v]), m);
-        }
-        AFSI_LAUNCH_CHECK();
-    }
+    for (int l = L.levels - 1; l >= 0; --l)
+        for (int c = 0; c < L.chunks[l]; ++c)
+            if (int r = batch_stage<P>(L, l, desc(l, L.chunks[l] + c), false, s)) return r;
     return OK;
 }
 

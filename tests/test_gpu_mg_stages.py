@@ -1,0 +1,48 @@
+"""The tiled smoothing stages of the 3D V-cycle against the oracle's cycle
+where tiles, halos and phase chunks can go wrong: extents that are no multiple
+of the tile, axes shorter than a tile with its halo, stages that need several
+launches, both smoothers and boundary types, and a level large enough for the
+two-phase launches."""
+import numpy as np
+import pytest
+import torch
+
+from afsi_gpu_amd.mac import MACGrid, MGOptions
+from afsi_gpu_amd.mac.multigrid import GeometricMultigrid
+from oracle import mac3d
+
+pytestmark = pytest.mark.gpu
+LENGTHS = (1., 1.3, .9)
+
+
+def check(gpu, shape, periodic, smoother, nu):
+    h = tuple(L / n for L, n in zip(LENGTHS, shape))
+    ref = mac3d.Multigrid(shape, h, mac3d.MGOptions(smooth=nu, smoother=smoother), periodic)
+    gen = np.random.default_rng(5)
+    start, rhs = gen.normal(size=shape), gen.normal(size=shape) / min(h) ** 2
+    start -= start.mean()
+    rhs -= rhs.mean()
+    want = ref.cycle(0, start, rhs)
+    want -= want.mean()
+    # an FP32 cycle rounds 2^29 times as coarsely; 2e-12 covers about 100
+    # FP64 roundings along any path of the cycle
+    for dtype, bound in ((torch.float64, 2e-12), (torch.float32, 2e-12 * 2. ** 29)):
+        mg = GeometricMultigrid(MACGrid(shape, LENGTHS, periodic=periodic), device=gpu, dtype=dtype,
+                                options=MGOptions(smooth=nu, smoother=smoother), backend='workspace')
+        mg.initialize(torch.tensor(start, device=gpu, dtype=dtype), torch.tensor(rhs, device=gpu, dtype=dtype))
+        got = mg.cycle().double().cpu().numpy()
+        got -= got.mean()
+        assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want), (shape, dtype)
+
+
+@pytest.mark.parametrize('periodic', [False, True], ids=['closed', 'periodic'])
+@pytest.mark.parametrize('smoother,nu', [('rbgs', 1), ('rbgs', 2), ('rbgs', 3), ('jacobi', 4), ('jacobi', 5)])
+@pytest.mark.parametrize('shape', [(24, 40, 48), (128, 16, 16), (12, 40, 40), (40, 56, 24)])
+def test_cycle_matches_oracle(gpu, shape, smoother, nu, periodic):
+    check(gpu, shape, periodic, smoother, nu)
+
+
+@pytest.mark.parametrize('periodic', [False, True], ids=['closed', 'periodic'])
+@pytest.mark.parametrize('smoother,nu', [('rbgs', 2), ('jacobi', 3)])
+def test_two_phase_level_matches_oracle(gpu, smoother, nu, periodic):
+    check(gpu, (128, 80, 112), periodic, smoother, nu)
