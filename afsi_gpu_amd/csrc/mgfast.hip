@@ -35,7 +35,7 @@ int launch_reduce_final(const double* partials, int64_t nparts, double* result, 
 
 constexpr int COARSE_THREADS = 1024;
 constexpr int64_t COARSE_MAX = 4096;  // cells of the finest level solved in LDS
-constexpr int COARSE_LIST = 4800;     // packed cell descriptors of all LDS levels
+constexpr int COARSE_TOTAL = 4800;    // cells of all LDS levels
 
 struct Dim32 {
     int n0, n1, n2;
@@ -888,263 +888,8 @@ __global__ void refine_update_kernel(double* __restrict__ x, const float* __rest
 // inv(A + 11^T/n) solve returns the mean of its right-hand side, so the
 // reference's mean subtractions change only rounding; the caller removes
 // the level-0 mean once after the last cycle.
-// Work items are enumerated per colour (lanes map to the red or the black
-// cells of rows directly) and decoded with float-reciprocal division plus
-// an exact integer correction; 1/diag comes from a per-level table.
 
-template <class T>
-struct CoarseArgs {
-    int32_t levels;  // number of levels handled (>= 1)
-    int32_t smoother, nu;
-    T omega;
-    Dim32 d[AFSI_MG_MAX_LEVELS];
-    W3<T> k[AFSI_MG_MAX_LEVELS];
-    int32_t off_p[AFSI_MG_MAX_LEVELS], off_r[AFSI_MG_MAX_LEVELS], off_w[AFSI_MG_MAX_LEVELS];
-    const T* rhs_in;   // first handled level's rhs (global)
-    const T* p_in;     // its initial iterate, or null (zero)
-    T* p_out;          // mean-free result of the first handled level
-    const T* coarse_inverse;
-    int32_t coarse_cells;
-    const int32_t* active;  // batched launches: skip when *active == 0 (null: always run)
-};
-
-// floor(e / d) for 0 <= e < 2^22, d >= 1
-__device__ inline int qdiv(int e, int d) {
-    int q = int((float(e) + 0.5f) / float(d));
-    if (q * d > e) --q;
-    else if ((q + 1) * d <= e) ++q;
-    return q;
-}
-
-// sum_nb w_a p_nb (and, for Neumann, the boundary class index) at (x,y,z).
-template <class T, bool P>
-__device__ inline T lds_nsum(const T* a, int i, int x, int y, int z, const Dim32& d,
-                             const W3<T>& k) {
-    const int sx = d.n1 * d.n2, sy = d.n2;
-    T s = T(0);
-    if (P) {
-        s += k.w[0] * a[i + (x + 1 < d.n0 ? sx : -(d.n0 - 1) * sx)];
-        s += k.w[0] * a[i + (x > 0 ? -sx : (d.n0 - 1) * sx)];
-        s += k.w[1] * a[i + (y + 1 < d.n1 ? sy : -(d.n1 - 1) * sy)];
-        s += k.w[1] * a[i + (y > 0 ? -sy : (d.n1 - 1) * sy)];
-        s += k.w[2] * a[i + (z + 1 < d.n2 ? 1 : -(d.n2 - 1))];
-        s += k.w[2] * a[i + (z > 0 ? -1 : (d.n2 - 1))];
-    } else {
-        if (x + 1 < d.n0) s += k.w[0] * a[i + sx];
-        if (x > 0) s += k.w[0] * a[i - sx];
-        if (y + 1 < d.n1) s += k.w[1] * a[i + sy];
-        if (y > 0) s += k.w[1] * a[i - sy];
-        if (z + 1 < d.n2) s += k.w[2] * a[i + 1];
-        if (z > 0) s += k.w[2] * a[i - 1];
-    }
-    return s;
-}
-
-template <class T, bool P>
-__device__ inline T lds_inv(const T* tab, T inv_p, int x, int y, int z, const Dim32& d) {
-    if (P) return inv_p;
-    return tab[face_class(x, d.n0) * 9 + face_class(y, d.n1) * 3 + face_class(z, d.n2)];
-}
-
-// Packed cell descriptor: x (bits 24-29), y (18-23), z (12-17), index (0-11).
-__device__ inline uint32_t pack_cell(int x, int y, int z, int i) {
-    return (uint32_t(x) << 24) | (uint32_t(y) << 18) | (uint32_t(z) << 12) | uint32_t(i);
-}
-__device__ inline void unpack_cell(uint32_t c, int& x, int& y, int& z, int& i) {
-    x = int(c >> 24);
-    y = int((c >> 18) & 63);
-    z = int((c >> 12) & 63);
-    i = int(c & 4095);
-}
-
-// Lists: for a level with even n2, cells of colour c (x+y+z even: red) at
-// list[c*n/2 + row*n2/2 + z/2]; otherwise all cells in index order.
-__device__ inline void build_list(uint32_t* list, const Dim32& d) {
-    const int n = d.n0 * d.n1 * d.n2;
-    const bool split = (d.n2 & 1) == 0;
-    for (int e = threadIdx.x; e < n; e += COARSE_THREADS) {
-        const int row = qdiv(e, d.n2), z = e - row * d.n2;
-        const int x = qdiv(row, d.n1), y = row - x * d.n1;
-        const uint32_t c = pack_cell(x, y, z, e);
-        if (split) list[((x + y + z) & 1) * (n >> 1) + row * (d.n2 >> 1) + (z >> 1)] = c;
-        else list[e] = c;
-    }
-}
-
-template <class T, bool P>
-__device__ inline void lds_smooth(T* p, T* w, const T* r, const uint32_t* list, const Dim32& d,
-                                  const W3<T>& k, const T* tab, T inv_p, int smoother, int nu,
-                                  T omega) {
-    const int n = d.n0 * d.n1 * d.n2;
-    const int sx = d.n1 * d.n2, sy = d.n2;
-    if (smoother == 1) {
-        const int half = n >> 1;
-        for (int it = 0; it < nu; ++it) {
-            for (int color = 0; color < 2; ++color) {
-                for (int e = threadIdx.x; e < half; e += COARSE_THREADS) {
-                    int x, y, z, i;
-                    unpack_cell(list[color * half + e], x, y, z, i);
-                    T s;
-                    if (P) {
-                        s = k.w[0] * p[i + (x + 1 < d.n0 ? sx : -(d.n0 - 1) * sx)];
-                        s += k.w[0] * p[i + (x > 0 ? -sx : (d.n0 - 1) * sx)];
-                        s += k.w[1] * p[i + (y + 1 < d.n1 ? sy : -(d.n1 - 1) * sy)];
-                        s += k.w[1] * p[i + (y > 0 ? -sy : (d.n1 - 1) * sy)];
-                        s += k.w[2] * p[i + (z + 1 < d.n2 ? 1 : -(d.n2 - 1))];
-                        s += k.w[2] * p[i + (z > 0 ? -1 : (d.n2 - 1))];
-                    } else {
-                        s = T(0);
-                        if (x + 1 < d.n0) s += k.w[0] * p[i + sx];
-                        if (x > 0) s += k.w[0] * p[i - sx];
-                        if (y + 1 < d.n1) s += k.w[1] * p[i + sy];
-                        if (y > 0) s += k.w[1] * p[i - sy];
-                        if (z + 1 < d.n2) s += k.w[2] * p[i + 1];
-                        if (z > 0) s += k.w[2] * p[i - 1];
-                    }
-                    p[i] = rb_relax(k, p[i], (r[i] + s) * lds_inv<T, P>(tab, inv_p, x, y, z, d));
-                }
-                __syncthreads();
-            }
-        }
-    } else {
-        for (int it = 0; it < nu; ++it) {
-            for (int e = threadIdx.x; e < n; e += COARSE_THREADS) {
-                int x, y, z, i;
-                unpack_cell(list[e], x, y, z, i);
-                const T a = apply_diff<T, P>(p, i, sx, sy, x, y, z, d, k);
-                w[i] = p[i] + omega * (r[i] - a) * lds_inv<T, P>(tab, inv_p, x, y, z, d);
-            }
-            __syncthreads();
-            for (int i = threadIdx.x; i < n; i += COARSE_THREADS) p[i] = w[i];
-            __syncthreads();
-        }
-    }
-}
-
-template <class T, bool P>
-__device__ __forceinline__ void coarse_cycle_body(const CoarseArgs<T>& a) {
-    extern __shared__ unsigned char smem_raw[];
-    T* smem = reinterpret_cast<T*>(smem_raw);
-    __shared__ T tabs[AFSI_MG_MAX_LEVELS][27];
-    __shared__ uint32_t lists[COARSE_LIST];
-    __shared__ int list_off[AFSI_MG_MAX_LEVELS];
-    const int L = a.levels;
-    // The first level's rhs and initial iterate (at most COARSE_MAX cells)
-    // are loaded into registers first, so the loads' latency overlaps the
-    // cell-list build; they reach LDS after it.
-    constexpr int LOADS = int(COARSE_MAX / COARSE_THREADS);
-    static_assert(LOADS * COARSE_THREADS == COARSE_MAX, "whole loads per thread");
-    T rv[LOADS], pv[LOADS];
-    {
-        const int n = a.d[0].n0 * a.d[0].n1 * a.d[0].n2;
-#pragma unroll
-        for (int q = 0; q < LOADS; ++q) {
-            const int i = int(threadIdx.x) + q * COARSE_THREADS;
-            rv[q] = i < n ? a.rhs_in[i] : T(0);
-            pv[q] = i < n && a.p_in ? a.p_in[i] : T(0);
-        }
-    }
-    if (threadIdx.x == 0) {
-        int off = 0;
-        for (int l = 0; l < L; ++l) {
-            list_off[l] = off;
-            off += a.d[l].n0 * a.d[l].n1 * a.d[l].n2;
-        }
-    }
-    if (!P && threadIdx.x < 27 * L) {
-        const int l = threadIdx.x / 27;
-        tabs[l][threadIdx.x - 27 * l] = inv_diag_entry<T>(threadIdx.x - 27 * l, a.k[l]);
-    }
-    __syncthreads();
-    for (int l = 0; l < L; ++l) build_list(lists + list_off[l], a.d[l]);
-    {
-        const int n = a.d[0].n0 * a.d[0].n1 * a.d[0].n2;
-        T* p = smem + a.off_p[0];
-        T* r = smem + a.off_r[0];
-#pragma unroll
-        for (int q = 0; q < LOADS; ++q) {
-            const int i = int(threadIdx.x) + q * COARSE_THREADS;
-            if (i < n) {
-                r[i] = rv[q];
-                p[i] = pv[q];
-            }
-        }
-        __syncthreads();
-    }
-    for (int l = 0; l < L - 1; ++l) {
-        const Dim32& d = a.d[l];
-        const W3<T>& k = a.k[l];
-        T* p = smem + a.off_p[l];
-        T* r = smem + a.off_r[l];
-        T* w = smem + a.off_w[l];
-        const T inv_p = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
-        lds_smooth<T, P>(p, w, r, lists + list_off[l], d, k, tabs[l], inv_p, a.smoother, a.nu, a.omega);
-        const Dim32& c = a.d[l + 1];
-        T* rc = smem + a.off_r[l + 1];
-        T* pc = smem + a.off_p[l + 1];
-        const uint32_t* clist = lists + list_off[l + 1];
-        const int nc = c.n0 * c.n1 * c.n2;
-        const int sx = d.n1 * d.n2, sy = d.n2;
-        for (int e = threadIdx.x; e < nc; e += COARSE_THREADS) {
-            int x, y, z, i;
-            unpack_cell(clist[e], x, y, z, i);
-            T v = T(0);
-            for (int aa = 0; aa < 2; ++aa)
-                for (int b = 0; b < 2; ++b)
-                    for (int cc = 0; cc < 2; ++cc) {
-                        const int fx = 2 * x + aa, fy = 2 * y + b, fz = 2 * z + cc;
-                        const int j = fx * sx + fy * sy + fz;
-                        v += r[j] - apply_diff<T, P>(p, j, sx, sy, fx, fy, fz, d, k);
-                    }
-            rc[i] = v * T(0.125);
-            pc[i] = T(0);
-        }
-        __syncthreads();
-    }
-    {
-        const Dim32& d = a.d[L - 1];
-        T* p = smem + a.off_p[L - 1];
-        const T* r = smem + a.off_r[L - 1];
-        const int m = a.coarse_cells;
-        // tpr threads per row (a power of two <= 64, inside one wave)
-        int tpr = 1;
-        while (tpr < 64 && tpr * 2 * m <= COARSE_THREADS) tpr *= 2;
-        const int lane = threadIdx.x % tpr;
-        for (int row0 = 0; row0 < m; row0 += COARSE_THREADS / tpr) {
-            const int row = row0 + threadIdx.x / tpr;
-            T s = T(0);
-            if (row < m)
-                for (int col = lane; col < m; col += tpr) s += a.coarse_inverse[row * m + col] * r[col];
-            for (int dd = tpr / 2; dd >= 1; dd >>= 1) s += __shfl_xor(s, dd, WAVE);
-            if (row < m && lane == 0) p[row] = s;
-        }
-        __syncthreads();
-    }
-    for (int l = L - 2; l >= 0; --l) {
-        const Dim32& d = a.d[l];
-        const W3<T>& k = a.k[l];
-        T* p = smem + a.off_p[l];
-        T* r = smem + a.off_r[l];
-        T* w = smem + a.off_w[l];
-        const T* pc = smem + a.off_p[l + 1];
-        const uint32_t* list = lists + list_off[l];
-        const int n = d.n0 * d.n1 * d.n2;
-        for (int e = threadIdx.x; e < n; e += COARSE_THREADS) {
-            int x, y, z, i;
-            unpack_cell(list[e], x, y, z, i);
-            p[i] = p[i] + prolong32<T, P>(pc, x, y, z, d.n0 / 2, d.n1 / 2, d.n2 / 2);
-        }
-        __syncthreads();
-        const T inv_p = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
-        lds_smooth<T, P>(p, w, r, list, d, k, tabs[l], inv_p, a.smoother, a.nu, a.omega);
-    }
-    {
-        const Dim32& d = a.d[0];
-        const int n = d.n0 * d.n1 * d.n2;
-        const T* p = smem + a.off_p[0];
-        for (int i = threadIdx.x; i < n; i += COARSE_THREADS) a.p_out[i] = p[i];
-    }
-}
+#include "mgcoarse.hpp"
 
 template <class T, bool P>
 __global__ void __launch_bounds__(COARSE_THREADS) coarse_cycle_kernel(CoarseArgs<T> a) {
@@ -1491,27 +1236,10 @@ struct FastRunner {
     }
 
     int coarse(int first, const T* p_in, T* p_out) const {
-        CoarseArgs<T> a{};
-        a.levels = pl.levels - first;
-        a.smoother = pl.smoother;
-        a.nu = pl.nu;
-        a.omega = T(pl.omega);
-        int32_t off = 0;
-        for (int j = 0; j < a.levels; ++j) {
-            const int l = first + j;
-            a.d[j] = D(l);
-            a.k[j] = K(l);
-            const int32_t n = int32_t(cells(l));
-            a.off_p[j] = off; off += n;
-            a.off_r[j] = off; off += n;
-            a.off_w[j] = off; off += (pl.smoother == 1 ? 0 : n);
-        }
-        const size_t bytes = size_t(off) * sizeof(T);
-        a.rhs_in = R(first);
+        CoarseArgs<T> a;
+        const size_t bytes = size_t(coarse_args<T>(pl, first, a)) * sizeof(T);
         a.p_in = p_in;
         a.p_out = p_out;
-        a.coarse_inverse = static_cast<const T*>(pl.coarse_inverse);
-        a.coarse_cells = int32_t(pl.coarse_cells);
         if (int r = dynamic_lds(pl.periodic ? reinterpret_cast<const void*>(coarse_cycle_kernel<T, true>)
                                             : reinterpret_cast<const void*>(coarse_cycle_kernel<T, false>),
                                 bytes))
@@ -1633,7 +1361,7 @@ struct FastRunner {
 };
 
 // First level solved by the LDS kernel: at most COARSE_MAX cells, every
-// extent <= 64, and all of its levels' cell lists within COARSE_LIST.
+// extent <= 64, and at most COARSE_TOTAL cells on all of its levels.
 static int choose_coarse(const afsi_mg3d_plan& pl) {
     for (int l = 0; l < pl.levels; ++l) {
         int64_t total = 0;
@@ -1642,7 +1370,7 @@ static int choose_coarse(const afsi_mg3d_plan& pl) {
             ok = pl.n[j][0] <= 64 && pl.n[j][1] <= 64 && pl.n[j][2] <= 64;
             total += pl.n[j][0] * pl.n[j][1] * pl.n[j][2];
         }
-        if (ok && total <= COARSE_LIST) return l;
+        if (ok && total <= COARSE_TOTAL) return l;
     }
     return -1;
 }
@@ -1791,9 +1519,9 @@ static int batch_layout(const afsi_mgb_batch* bt, BatchLayout& L) {
     L.ref_blocks = 0;
     for (int i = 0; i < L.n; ++i) {
         const afsi_mg3d_plan& pl = bt->items[i].plan;
-        size_t cells = 0;
-        for (int l = L.cf[i]; l < pl.levels; ++l) cells += 2 * size_t(pl.n[l][0] * pl.n[l][1] * pl.n[l][2]);
-        if (cells * sizeof(float) > L.coarse_lds) L.coarse_lds = cells * sizeof(float);
+        CoarseArgs<float> a;
+        const size_t bytes = size_t(coarse_args<float>(pl, L.cf[i], a)) * sizeof(float);
+        if (bytes > L.coarse_lds) L.coarse_lds = bytes;
         L.ref_blocks += int(cdiv(pl.n[0][0] * pl.n[0][1], 4));
     }
     for (int v = 0; v < 4; ++v) {
@@ -1864,28 +1592,10 @@ static int batch_prepare(const afsi_mgb_batch* bt, hipStream_t s) {
     for (int i = 0; i < L.n; ++i) {
         const afsi_mgb_item& it = bt->items[i];
         const afsi_mg3d_plan& pl = it.plan;
-        CoarseArgs<float> a{};
+        CoarseArgs<float> a;
         const int first = L.cf[i];
-        a.levels = pl.levels - first;
-        a.smoother = pl.smoother;
-        a.nu = pl.nu;
-        a.omega = float(pl.omega);
-        int32_t o = 0;
-        for (int j = 0; j < a.levels; ++j) {
-            const int l = first + j;
-            a.d[j] = Dim32{int(pl.n[l][0]), int(pl.n[l][1]), int(pl.n[l][2])};
-            for (int q = 0; q < 3; ++q) a.k[j].w[q] = float(pl.inv_h2[l][q]);
-            a.k[j].relax = float(pl.relax > 0.0 ? pl.relax : 1.0);
-            const int32_t c = int32_t(pl.n[l][0] * pl.n[l][1] * pl.n[l][2]);
-            a.off_p[j] = o; o += c;
-            a.off_r[j] = o; o += c;
-            a.off_w[j] = o;
-        }
-        a.rhs_in = static_cast<const float*>(pl.rhs[first]);
+        coarse_args<float>(pl, first, a);
         a.p_in = nullptr;  // zero initial guess on every level
-        a.p_out = static_cast<float*>(pl.p[first]);
-        a.coarse_inverse = static_cast<const float*>(pl.coarse_inverse);
-        a.coarse_cells = int32_t(pl.coarse_cells);
         a.active = bt->active + i;
         at<CoarseArgs<float>>(hw, L.coarse_off[0])[i] = a;
         // a later cycle of one refinement iteration continues from the
