@@ -161,8 +161,11 @@ class ChannelMultigrid:
         return self.p[0]
 
     @torch.no_grad()
-    def solve(self, rhs, initial=None, *, history=None):
-        """mac2d/multigrid.py:83-134 (workspace branch :111-134)."""
+    def solve(self, rhs, initial=None, *, history=None, precheck=None):
+        """mac2d/multigrid.py:83-134 (workspace branch :111-134). ``precheck``,
+        if given, is called right after the first host synchronisation, before
+        any cycle and before the RHS checks: a caller can read there device
+        flags that it copied to pinned memory earlier on the stream."""
         if rhs.shape != self.shapes[0] or rhs.device != self.device or rhs.dtype != self.dtype:
             raise ValueError('invalid channel pressure RHS')
         if initial is not None and (initial.shape != rhs.shape or initial.dtype != rhs.dtype
@@ -183,6 +186,8 @@ class ChannelMultigrid:
         _abi.call(f'afsi_mg2d_residual_{self.suffix}', self.plan, _abi.stream())
         (s1, _, a1, nf1), (_, _, _, nf2), (_, q3, _, _), (_, q0, _, nf0) = \
             self.results[[1, 2, 3, 0]].tolist()
+        if precheck is not None:
+            precheck()
         if nf1 or nf2:
             raise ValueError('finite pressure RHS/initial guess required')
         count = w_rhs.numel()

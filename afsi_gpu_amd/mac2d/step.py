@@ -2,11 +2,15 @@
 with the point force given): prepare -> spread -> u* = u + (dt/rho) f with
 the wall normal faces kept at zero and the inlet face kept at its value
 (the boundary() of mac2d/grid.py:74-79) -> project -> gather -> x += dt U.
+
+The checks of the parts (support of the points, finite tentative velocity)
+are made on the device and read at the pressure solve's first
+synchronisation, before anything of the caller's is changed.
 """
 import torch
 
-from .flow import ChannelFlow
 from . import transfer
+from .flow import ChannelFlow, ChannelResult, correct, divergence
 
 
 class ChannelIBStep:
@@ -18,17 +22,42 @@ class ChannelIBStep:
     @torch.no_grad()
     def step(self, x, force, velocity, pressure=None, *, advance=True):
         """Returns (velocity, pressure, point_velocity, info); x advances in place."""
-        stencil = transfer.prepare(self.grid, x)
-        density = transfer.spread(self.grid, force, stencil)
+        # this call's own device word: a stepper may be shared by several streams
+        flags = torch.zeros((), dtype=torch.int32, device=x.device)
+        host = torch.empty((), dtype=torch.int32, pin_memory=True)
+        stencil = transfer.prepare(self.grid, x, flags=flags)
+        host.copy_(flags, non_blocking=True)
+        density = transfer.spread(self.grid, force, stencil, check=False)
         coef = self.dt / self.rho
-        u = velocity[0] + coef * density[0]
-        v = velocity[1] + coef * density[1]
+        u = torch.add(velocity[0], density[0], alpha=coef)
+        v = torch.add(velocity[1], density[1], alpha=coef)
         if not self.grid.periodic:
             u[0] = velocity[0][0]
         v[:, 0] = 0
         v[:, -1] = 0
-        result = self.flow.project((u, v), pressure)
-        U = transfer.gather(self.grid, result.velocity, stencil)
+        result = self._project((u, v), pressure, host)
+        U = transfer.gather(self.grid, result.velocity, stencil, check=False)
         if advance:
             x.add_(U, alpha=self.dt)
         return result.velocity, result.pressure, U, result.diagnostics
+
+    def _project(self, tentative, pressure, host):
+        """ChannelFlow.project of velocities that are this step's own (corrected
+        in place, wall faces already zero), its checks deferred: a nonfinite
+        face makes the right-hand side nonfinite, which the solve rejects."""
+        flow = self.flow
+        self.grid.check_velocity(tentative)
+
+        def precheck():
+            if int(host) & 1:
+                raise ValueError(transfer.SUPPORT_MESSAGE)
+
+        rhs = divergence(tentative, self.grid, -flow.rho / flow.dt, out=flow._rhs)
+        try:
+            p, info = flow.pressure_solver.solve(rhs, pressure, precheck=precheck)
+        except ValueError:
+            if not int(host) & 1 and any(not torch.isfinite(t).all() for t in tentative):
+                raise ValueError('finite tentative velocity required') from None
+            raise
+        velocity = correct(tentative, p, self.grid, flow.dt / flow.rho)
+        return ChannelResult(velocity, p, dict(pressure=info))

@@ -20,8 +20,16 @@ class Stencil:
     weights: tuple
 
 
-def prepare(grid, points):
-    """mac2d/transfer.py:83-101: support check, then the reflected stencil."""
+SUPPORT_MESSAGE = 'valve IB points leave the channel support region'
+
+
+def prepare(grid, points, *, flags=None):
+    """mac2d/transfer.py:83-101: support check, then the reflected stencil.
+
+    ``flags``: a zeroed int32 device word the kernel ORs its error bits into
+    (1: a point outside the support region; its links then carry weight
+    zero). The caller reads it, so nothing synchronises here; by default the
+    check is made at once."""
     cuda_ib.require_cuda(points)
     if points.dim() != 2 or points.shape[1] != 2 or points.dtype != torch.float64:
         raise ValueError('channel IB points must be (P,2) float64')
@@ -30,26 +38,30 @@ def prepare(grid, points):
     kw = dict(device=points.device)
     ids = [torch.empty((P, 16), dtype=torch.int64, **kw) for _ in range(2)]
     w = [torch.empty((P, 16), dtype=torch.float64, **kw) for _ in range(2)]
-    flags = torch.zeros((), dtype=torch.int32, **kw)
+    check = flags is None
+    if check:
+        flags = torch.zeros((), dtype=torch.int32, **kw)
     g = grid.abi()
     _abi.call('afsi_channel_prepare_f64', _abi.ptr(points), P, g, _abi.ptr(ids[0]), _abi.ptr(w[0]),
               _abi.ptr(ids[1]), _abi.ptr(w[1]), _abi.ptr(flags), _abi.stream())
-    if int(flags.item()) & 1:
-        raise ValueError('valve IB points leave the channel support region')
+    if check and int(flags.item()) & 1:
+        raise ValueError(SUPPORT_MESSAGE)
     return Stencil(tuple(ids), tuple(w))
 
 
-def spread(grid, force, stencil):
-    """Face densities f_c = sum (F_c w)/V per component (mac2d/transfer.py:108-115)."""
+def spread(grid, force, stencil, *, check=True):
+    """Face densities f_c = sum (F_c w)/V per component (mac2d/transfer.py:108-115).
+    ``check=False`` skips the index check's host synchronisations (ids made by
+    ``prepare`` for the same grid are in range)."""
     cuda_ib.require_cuda(force)
     force = force.contiguous()
     return tuple(cuda_ib.indexed_spread(force[:, c:c + 1].contiguous(), stencil.indices[c],
                                         stencil.weights[c], grid.face_shape(c)[0] *
-                                        grid.face_shape(c)[1], grid.volume).reshape(grid.face_shape(c))
+                                        grid.face_shape(c)[1], grid.volume, check=check).reshape(grid.face_shape(c))
                  for c in range(2))
 
 
-def gather(grid, velocity, stencil):
-    """U[p, c] = sum_k u_c[ids] w (mac2d/transfer.py:123-127)."""
-    return torch.cat([cuda_ib.indexed_gather(u.reshape(-1, 1), ids, w)
+def gather(grid, velocity, stencil, *, check=True):
+    """U[p, c] = sum_k u_c[ids] w (mac2d/transfer.py:123-127); ``check`` as for ``spread``."""
+    return torch.cat([cuda_ib.indexed_gather(u.reshape(-1, 1), ids, w, check=check)
                       for u, ids, w in zip(velocity, stencil.indices, stencil.weights)], -1)
