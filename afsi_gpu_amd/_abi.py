@@ -270,6 +270,13 @@ _SIGNATURES = {
     'afsi_chb_spread_f64': (c_int, [POINTER(CHBBatch), _P, _P, _P, _P, c_size_t, _P, _P]),
     'afsi_p1_contract_f64': (c_int, [POINTER(FEGeometry), _P, _P, c_int64, c_int64, c_int, POINTER(Grid3),
                                      POINTER(HashTable), _P]),
+    'afsi_p1_row_sites_limit': (c_int64, []),
+    'afsi_p1_row_boxes_f64': (c_int, [POINTER(FEGeometry), _P, POINTER(Grid3), _P, _P, _P, _P, _P, _P]),
+    'afsi_p1_rows_f64': (c_int, [POINTER(FEGeometry), _P, POINTER(Grid3), _P, _P, _P, _P, c_int64, _P, _P, _P, _P,
+                                 _P]),
+    'afsi_p1_rows_csr_workspace_bytes': (c_size_t, [POINTER(Grid3), c_int64]),
+    'afsi_p1_rows_csr_f64': (c_int, [POINTER(Grid3), c_int64, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P,
+                                     c_size_t, _P]),
     'afsi_csr_spmv_f64': (c_int, [POINTER(CSR), _P, c_int64, _P, c_int64, c_double, _P]),
 }
 

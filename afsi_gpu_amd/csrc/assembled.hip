@@ -4,7 +4,9 @@
 // contracted per cell (mac/csrc/ib.cu:56-123) and reduced over cells in a
 // bounded open-addressing table keyed by node * faces + face
 // (mac/hash_transfer_assembly.py:13-70): SplitMix64 finaliser buckets,
-// linear probing of at most 128 slots, empty key -1, overflow -> flag.
+// linear probing of at most 128 slots, empty key -1, overflow -> flag. The
+// table takes single components, callers' own entries and rows too large for
+// LDS; whole operators are otherwise assembled by rows (assembled_rows.hip).
 // Spread and interpolation are then CSR products (csr_spmv below).
 //
 // Contraction: one wave per cell. The cell's stencil box of component c

@@ -7,13 +7,18 @@ operator of mac/assembled_transfer.py:1-8 and :138-211
 built once per ``prepare`` and then applied by CSR products in both
 directions: spread = B_c^T (M^-1 b) / V, interpolation solves M U = B u.
 
-Construction per component (``csrc/assembled.hip``): the cells are
-contracted in parallel, one wave per cell accumulating its stencil box in
-LDS, into a bounded device hash table (``HashWorkspace``; a probe overflow
-discards the whole table and retries at twice the capacity, up to the
-entry budget, mac/hash_transfer_assembly.py:132-155); the occupied keys are
-then sorted once and split into the node-major CSR B and its face-major
-transpose. Only the table's flag and the entry count reach the host.
+Construction (``csrc/assembled_rows.hip``): one wave per node and component
+accumulates the node's row in LDS and writes its nonzeros in face order; the
+transpose comes from one 32-bit stable sort by face. Two host reads: the
+rows' box sizes and the entry counts.
+
+Where a row's stencil box exceeds LDS (cells many faces wide) the cells are
+contracted per component (``csrc/assembled.hip``), one wave per cell, into a
+bounded device hash table (``HashWorkspace``; a probe overflow discards the
+whole table and retries at twice the capacity, up to the entry budget,
+mac/hash_transfer_assembly.py:132-155); the occupied keys are then sorted and
+split into the node-major CSR B and its face-major transpose. The ``hash_*``
+statistics are 0 for components assembled by rows.
 """
 from dataclasses import dataclass
 from math import prod
@@ -160,17 +165,78 @@ class AssembledTransfer(FETransfer):
         return B, BT, dict(raw_cell_entries=raw, nnz=len(keys), hash_capacity=capacity, hash_attempts=attempts,
                            hash_workspace_bytes=workspace.storage_bytes)
 
-    @torch.no_grad()
-    def assemble_stencil(self, points):
-        stencil = from_points(points.contiguous(), self.grid, check=False)
+    def _rows(self, base, phi):
+        """The three components by rows, or None where a row's stencil box
+        does not fit (the hash table takes those)."""
+        g, A = self.geometry, self.geometry.cells.shape[1]
+        (E, Q), N = g.weights.shape, g.node_count
+        shapes = [self.grid.face_shape(c) for c in range(3)]
+        faces = [prod(shape) for shape in shapes]
+        limit = _abi.load().afsi_p1_row_sites_limit()
+        if Q > 64 or sum(faces) >= 2 ** 31 - 3 or max(E, N) >= 2 ** 28:
+            return None
+        grid, device = self.grid.abi(), g.weights.device
+        empty = lambda *shape, dtype=torch.int32: torch.empty(shape, dtype=dtype, device=device)
+        chunks, cell_box, row_box = empty(3, E, 64, dtype=torch.int64), empty(3, E, 6), empty(3 * N, 6)
+        sites, counts = empty(3 * N, dtype=torch.int64), empty(3 * N, dtype=torch.int64)
+        stats = torch.zeros(5, dtype=torch.int64, device=device)
+        _abi.call('afsi_p1_row_boxes_f64', self._g, _abi.ptr(base), grid, _abi.ptr(chunks), _abi.ptr(cell_box),
+                  _abi.ptr(row_box), _abi.ptr(sites), _abi.ptr(stats), _abi.stream())
+        site_ptr = torch.cumsum(sites, 0)
+        *raw, largest, flag, total = torch.cat((stats, site_ptr[-1:])).tolist()
+        if flag & 2:
+            raise ValueError('invalid P1 cell table or stencil box for the assembled operator')
+        # four sites per budgeted entry bound the scratch of the rows; the
+        # table decides about emptier ones
+        if flag or largest > limit or total > 4 * self.max_entries:
+            return None
+        cols, vals = empty(max(1, total)), empty(max(1, total), dtype=torch.float64)
+        _abi.call('afsi_p1_rows_f64', self._g, _abi.ptr(phi), grid, _abi.ptr(chunks), _abi.ptr(cell_box),
+                  _abi.ptr(row_box), _abi.ptr(site_ptr), max(512, largest), _abi.ptr(cols), _abi.ptr(vals),
+                  _abi.ptr(counts), _abi.ptr(stats), _abi.stream())
+        row_end = torch.cumsum(counts, 0)
+        *ends, flag = torch.cat((row_end[N - 1::N], stats[4:])).tolist()
+        if ends[2] > self.max_entries:
+            raise RuntimeError('assembled IB entry budget exceeded; no hash entries were truncated')
+        if flag:
+            raise FloatingPointError('invalid hash IB entries: nonfinite values')
+        nnz = ends[2]
+        if nnz >= 2 ** 31:
+            raise RuntimeError('assembled IB entry budget exceeded')
+        row_ptr, b_cols, b_vals = empty(3, N + 1), empty(nnz), empty(nnz, dtype=torch.float64)
+        face_ptr, t_cols, t_vals = empty(sum(faces) + 3), empty(nnz), empty(nnz, dtype=torch.float64)
+        size = _abi.load().afsi_p1_rows_csr_workspace_bytes(grid, nnz)
+        work = empty(size, dtype=torch.uint8)
+        _abi.call('afsi_p1_rows_csr_f64', grid, N, nnz, _abi.ptr(site_ptr), _abi.ptr(row_end), _abi.ptr(cols),
+                  _abi.ptr(vals), _abi.ptr(row_ptr), _abi.ptr(b_cols), _abi.ptr(b_vals), _abi.ptr(face_ptr),
+                  _abi.ptr(t_cols), _abi.ptr(t_vals), _abi.ptr(work), size, _abi.stream())
+        gather, spread, info = [], [], []
+        first = start = 0
+        for c, (end, nf) in enumerate(zip(ends, faces)):
+            part = slice(first, end)
+            gather.append(CSRMatrix(row_ptr[c], b_cols[part], b_vals[part], N))
+            spread.append(CSRMatrix(face_ptr[start:start + nf + 1], t_cols[part], t_vals[part], nf))
+            info.append(dict(raw_cell_entries=raw[c] * A, nnz=end - first, hash_capacity=0, hash_attempts=0,
+                             hash_workspace_bytes=0))
+            first, start = end, start + nf + 1
+        return gather, spread, info
+
+    def _hashed(self, base, phi):
         gather, spread, stats = [], [], []
         remaining = self.max_entries
         for c in range(3):
-            B, BT, info = self._component(c, stencil.base, stencil.phi, remaining)
+            B, BT, info = self._component(c, base, phi, remaining)
             remaining -= info['nnz']
             gather.append(B)
             spread.append(BT)
             stats.append(info)
+        return gather, spread, stats
+
+    @torch.no_grad()
+    def assemble_stencil(self, points):
+        stencil = from_points(points.contiguous(), self.grid, check=False)
+        gather, spread, stats = (self._rows(stencil.base, stencil.phi) or
+                                 self._hashed(stencil.base, stencil.phi))
         self.csr_builds += 1
         return AssembledStencil(tuple(gather), tuple(spread),
                                 dict(components=stats, total_nnz=sum(s['nnz'] for s in stats),

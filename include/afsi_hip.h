@@ -782,6 +782,35 @@ int afsi_hash_accumulate_f64(const int64_t* keys, const double* values, int64_t 
 int afsi_p1_contract_f64(const afsi_fe_geometry* g, const int64_t* base, const double* phi, int64_t lattice_points,
                          int64_t offset, int component, const afsi_grid3* grid, const afsi_hash_table* t,
                          void* stream);
+/* The same operator for all three components at once, by rows: no table, no
+ * order-dependent sums. Cells of at most 4 nodes and 64 points, closed boxes.
+ * Step 1, boxes: chunks (3,E,64) uint64 lists each cell's points by
+ * stencil base, four to a chunk, cell_box (3,E,6) and row_box (3*nodes,6) are stencil boxes, sites
+ * (3*nodes) the rows' box sizes. stats (5) int64, zero on entry: box sites of
+ * all cells per component, largest row box if it exceeds 512, flag (1: a
+ * cell's bases span more than 256 faces, 2: invalid cell table or stencil
+ * box; the row boxes are not written then, 4: nonfinite entry, set by step
+ * 2). */
+int64_t afsi_p1_row_sites_limit(void);
+int afsi_p1_row_boxes_f64(const afsi_fe_geometry* g, const int64_t* base, const afsi_grid3* grid, uint64_t* chunks,
+                          int32_t* cell_box, int32_t* row_box, int64_t* sites, int64_t* stats, void* stream);
+/* Step 2, rows: nonzeros of row r in face order at cols / vals +
+ * site_ptr[r-1] (site_ptr: inclusive sums of sites), their number in
+ * counts[r]. max_sites bounds every row's sites and is at most
+ * afsi_p1_row_sites_limit(). */
+int afsi_p1_rows_f64(const afsi_fe_geometry* g, const double* phi, const afsi_grid3* grid, const uint64_t* chunks,
+                     const int32_t* cell_box, const int32_t* row_box, const int64_t* site_ptr, int64_t max_sites,
+                     int32_t* cols, double* vals, int64_t* counts, int64_t* stats, void* stream);
+/* Step 3, CSR: row_end = inclusive sums of counts, nnz = its last. The three
+ * node-major matrices one after the other (row_ptr (3,nodes+1), cols, vals)
+ * and the face-major transposes (face_ptr: faces_c + 1 pointers per
+ * component, face_nodes, face_vals); pointers count from the component's
+ * first entry. */
+size_t afsi_p1_rows_csr_workspace_bytes(const afsi_grid3* grid, int64_t nnz);
+int afsi_p1_rows_csr_f64(const afsi_grid3* grid, int64_t nodes, int64_t nnz, const int64_t* site_ptr,
+                         const int64_t* row_end, const int32_t* cols_in, const double* vals_in, int32_t* row_ptr,
+                         int32_t* cols, double* vals, int32_t* face_ptr, int32_t* face_nodes, double* face_vals,
+                         void* workspace, size_t workspace_bytes, void* stream);
 /* y[r * y_stride] = scale * sum_k A[r, cols[k]] x[cols[k] * x_stride]: the
  * CSR products of the assembled spread (B^T c / V) and gather (B u) of
  * mac/assembled_transfer.py:199-211 (torch.sparse.mm). */
