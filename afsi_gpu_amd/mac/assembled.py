@@ -201,8 +201,8 @@ class AssembledTransfer(FETransfer):
         if flag:
             raise FloatingPointError('invalid hash IB entries: nonfinite values')
         nnz = ends[2]
-        if nnz >= 2 ** 31:
-            raise RuntimeError('assembled IB entry budget exceeded')
+        if nnz >= 2 ** 31:  # the entries of all components are sorted together
+            return None
         row_ptr, b_cols, b_vals = empty(3, N + 1), empty(nnz), empty(nnz, dtype=torch.float64)
         face_ptr, t_cols, t_vals = empty(sum(faces) + 3), empty(nnz), empty(nnz, dtype=torch.float64)
         size = _abi.load().afsi_p1_rows_csr_workspace_bytes(grid, nnz)

@@ -738,7 +738,7 @@ def main():
                            'algorithmic bytes 48 per point + 24 per cell'),
         roofline_sweep=dict(bound='hbm', achieved=achieved / 1e9, peak=HBM_PEAK / 1e9, unit='GB/s',
                             frac=achieved / HBM_PEAK, traffic=measured_traffic(n),
-                            kernel='rb_rows_kernel<float,true,4,4> (level-0 sweep, 24 launches per mixed step)',
+                            kernel='rb_rows_kernel<float,true,4,4> (level-0 sweep through the sweep entry point)',
                             algorithmic_bytes=sweep_bytes, avg_us=sweep_s * 1e6),
         plain_fp64=dict(steps_per_s=plain['steps_per_s'], ms_per_step=plain['ms_per_step'],
                         phases_ms=plain['phases_ms'], mg_cycles_mean=plain['mg_cycles_mean'],
