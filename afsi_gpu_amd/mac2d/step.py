@@ -29,8 +29,9 @@ class ChannelIBStep:
         host.copy_(flags, non_blocking=True)
         density = transfer.spread(self.grid, force, stencil, check=False)
         coef = self.dt / self.rho
-        u = torch.add(velocity[0], density[0], alpha=coef)
-        v = torch.add(velocity[1], density[1], alpha=coef)
+        # row-major whatever the caller's strides: the projection passes pointers
+        u = torch.add(velocity[0], density[0], alpha=coef).contiguous()
+        v = torch.add(velocity[1], density[1], alpha=coef).contiguous()
         if not self.grid.periodic:
             u[0] = velocity[0][0]
         v[:, 0] = 0
