@@ -22,42 +22,49 @@ class ChannelIBStep:
     @torch.no_grad()
     def step(self, x, force, velocity, pressure=None, *, advance=True):
         """Returns (velocity, pressure, point_velocity, info); x advances in place."""
-        # this call's own device word: a stepper may be shared by several streams
-        flags = torch.zeros((), dtype=torch.int32, device=x.device)
-        host = torch.empty((), dtype=torch.int32, pin_memory=True)
+        flags = torch.zeros((), dtype=torch.int32, device=x.device)  # this call's own device word
         stencil = transfer.prepare(self.grid, x, flags=flags)
+        host = torch.empty((), dtype=torch.int32, pin_memory=True)
         host.copy_(flags, non_blocking=True)
-        density = transfer.spread(self.grid, force, stencil, check=False)
-        coef = self.dt / self.rho
-        # row-major whatever the caller's strides: the projection passes pointers
-        u = torch.add(velocity[0], density[0], alpha=coef).contiguous()
-        v = torch.add(velocity[1], density[1], alpha=coef).contiguous()
-        if not self.grid.periodic:
-            u[0] = velocity[0][0]
-        v[:, 0] = 0
-        v[:, -1] = 0
-        result = self._project((u, v), pressure, host)
+        read = []
+
+        def precheck():  # after the solve's first synchronisation: the copy has arrived
+            read.append(int(host))
+            if read[0] & 1:
+                raise ValueError(transfer.SUPPORT_MESSAGE)
+
+        try:
+            density = transfer.spread(self.grid, force, stencil, check=False)
+            coef = self.dt / self.rho
+            # row-major whatever the caller's strides: the projection passes pointers
+            u = torch.add(velocity[0], density[0], alpha=coef).contiguous()
+            v = torch.add(velocity[1], density[1], alpha=coef).contiguous()
+            if not self.grid.periodic:
+                u[0] = velocity[0][0]
+            v[:, 0] = 0
+            v[:, -1] = 0
+            result = self._project((u, v), pressure, precheck)
+        except Exception:
+            # a point outside the support comes before any other fault
+            if int(read[0] if read else flags) & 1:
+                raise ValueError(transfer.SUPPORT_MESSAGE) from None
+            raise
         U = transfer.gather(self.grid, result.velocity, stencil, check=False)
         if advance:
             x.add_(U, alpha=self.dt)
         return result.velocity, result.pressure, U, result.diagnostics
 
-    def _project(self, tentative, pressure, host):
+    def _project(self, tentative, pressure, precheck):
         """ChannelFlow.project of velocities that are this step's own (corrected
         in place, wall faces already zero), its checks deferred: a nonfinite
         face makes the right-hand side nonfinite, which the solve rejects."""
         flow = self.flow
         self.grid.check_velocity(tentative)
-
-        def precheck():
-            if int(host) & 1:
-                raise ValueError(transfer.SUPPORT_MESSAGE)
-
         rhs = divergence(tentative, self.grid, -flow.rho / flow.dt, out=flow._rhs)
         try:
             p, info = flow.pressure_solver.solve(rhs, pressure, precheck=precheck)
         except ValueError:
-            if not int(host) & 1 and any(not torch.isfinite(t).all() for t in tentative):
+            if any(not torch.isfinite(t).all() for t in tentative):
                 raise ValueError('finite tentative velocity required') from None
             raise
         velocity = correct(tentative, p, self.grid, flow.dt / flow.rho)

@@ -1,4 +1,6 @@
-"""ChannelIBStep with inputs a caller may pass: velocities of any stride order."""
+"""ChannelIBStep with inputs a caller may pass: velocities of any stride order
+and several faults at once (the support of the points is reported first,
+whatever else is wrong)."""
 import pytest
 import torch
 
@@ -36,3 +38,27 @@ def test_velocity_strides_do_not_matter(gpu, periodic, which):
     assert torch.equal(pa, pb) and torch.equal(Ua, Ub) and torch.equal(xa, xb)
     assert all(torch.equal(a, b) and b.is_contiguous() for a, b in zip(va, vb))
     assert all(torch.equal(a, b) for a, b in zip(velocity, kept))
+
+
+@pytest.mark.parametrize('other', ['pressure shape', 'pressure dtype', 'velocity shape', 'force', 'force shape'])
+def test_support_is_reported_first(gpu, other):
+    grid, stepper, x, force, velocity = setup(gpu, False)
+    pressure = torch.zeros(grid.shape, device=gpu, dtype=torch.float64)
+    if other == 'pressure shape':
+        pressure = pressure[:-1]
+    elif other == 'pressure dtype':
+        pressure = pressure.float()
+    elif other == 'velocity shape':
+        velocity[0] = velocity[0][:, :-1]
+    elif other == 'force':
+        force = torch.full_like(force, float('nan'))
+    else:
+        force = force[:-1]
+    for inside in (False, True):
+        if not inside:
+            x[5, 1] = -1.
+        else:
+            x[5, 1] = .5
+        with pytest.raises((ValueError, RuntimeError)) as error:
+            stepper.step(x, force, velocity, pressure)
+        assert ('support region' in str(error.value)) == (not inside)
