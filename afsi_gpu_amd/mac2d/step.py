@@ -18,10 +18,14 @@ class ChannelIBStep:
         self.grid, self.dt, self.rho = grid, float(dt), float(rho)
         self.flow = ChannelFlow(grid, dt=dt, rho=rho, device=device, options=options,
                                 pressure_backend=pressure_backend)
+        self._done = torch.cuda.Event()
 
     @torch.no_grad()
     def step(self, x, force, velocity, pressure=None, *, advance=True):
-        """Returns (velocity, pressure, point_velocity, info); x advances in place."""
+        """Returns (velocity, pressure, point_velocity, info); x advances in
+        place. The step returns with its last launches queued on the current
+        stream. Calls may come on different streams, one after the other (the
+        solver's buffers are shared, so not from two threads at once)."""
         flags = torch.zeros((), dtype=torch.int32, device=x.device)  # this call's own device word
         stencil = transfer.prepare(self.grid, x, flags=flags)
         host = torch.empty((), dtype=torch.int32, pin_memory=True)
@@ -43,7 +47,9 @@ class ChannelIBStep:
                 u[0] = velocity[0][0]
             v[:, 0] = 0
             v[:, -1] = 0
+            torch.cuda.current_stream(x.device).wait_event(self._done)  # the last step's use of the solver
             result = self._project((u, v), pressure, precheck)
+            self._done.record(torch.cuda.current_stream(x.device))
         except Exception:
             # a point outside the support comes before any other fault
             if int(read[0] if read else flags) & 1:

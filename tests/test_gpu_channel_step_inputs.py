@@ -1,6 +1,6 @@
-"""ChannelIBStep with inputs a caller may pass: velocities of any stride order
-and several faults at once (the support of the points is reported first,
-whatever else is wrong)."""
+"""ChannelIBStep with inputs a caller may pass: velocities of any stride order,
+several faults at once (the support of the points is reported first, whatever
+else is wrong), and one stepper called from several streams."""
 import pytest
 import torch
 
@@ -62,3 +62,34 @@ def test_support_is_reported_first(gpu, other):
         with pytest.raises((ValueError, RuntimeError)) as error:
             stepper.step(x, force, velocity, pressure)
         assert ('support region' in str(error.value)) == (not inside)
+
+
+def test_one_stepper_on_two_streams(gpu):
+    """A step returns with its last launches queued; the next call on another
+    stream works in the same solver buffers."""
+    grid, stepper, x, force, velocity = setup(gpu, True)
+    _, _, x2, force2, velocity2 = setup(gpu, True, seed=8)
+    want = [stepper.step(a.clone(), f, tuple(v))[:3] for a, f, v in ((x, force, velocity), (x2, force2, velocity2))]
+    torch.cuda.synchronize()
+    solver = stepper.flow.pressure_solver
+    sub_mean = solver._sub_mean
+    slow = [False]
+
+    def late(t, slot):  # the mean removals of a solve, held back on their stream
+        if slow[0] and t is solver.p[0]:
+            torch.cuda._sleep(20_000_000)
+        sub_mean(t, slot)
+
+    solver._sub_mean = late
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    args = [(x.clone(), force, tuple(velocity)), (x2.clone(), force2, tuple(velocity2))]
+    got = []
+    torch.cuda.synchronize()
+    for stream, a, delay in zip(streams, args, (True, False)):
+        slow[0] = delay
+        with torch.cuda.stream(stream):
+            got.append(stepper.step(*a)[:3])
+    torch.cuda.synchronize()
+    for (va, pa, Ua), (vb, pb, Ub) in zip(want, got):
+        assert torch.equal(pa, pb) and torch.equal(Ua, Ub)
+        assert all(torch.equal(a, b) for a, b in zip(va, vb))
