@@ -16,10 +16,12 @@
 //     LDS, for as many cycles as asked when level 0 itself fits.
 // Measured figures stand at channel_cycles in channel.hip.
 //
-// Updates use the Gauss-Seidel form (b + sum w nb) / diag with zero ghosts
-// where a neighbour is missing, and 1/diag from a nine-entry table (low end,
-// interior, high end of each axis). The restricted residual keeps the
-// difference form. The periodic channel's means are not removed inside a
+// Updates and the restricted residual use the difference form
+// p + omega (b - sum w (p - nb)) / diag, with 1/diag from a nine-entry table
+// (low end, interior, high end of each axis). Differences of neighbours are
+// nearly exact and the quotient is a small correction, so a stored value
+// carries little more than its own rounding; in the form (b + sum w nb) / diag
+// the residual stagnates 1.45 to 3 times higher. The periodic channel's means are not removed inside a
 // cycle: A 1 = 0, smoothing, restriction and prolongation commute with a
 // constant shift and the coarse inverse of a zero-mean residual has zero mean,
 // so the driver removes the mean of p once after the last cycle.
@@ -64,22 +66,30 @@ __device__ inline T chf_diag(int cx, int cy, const Coef2<T>& k) {
 
 __device__ inline int chf_class(int i, int n) { return i == 0 ? 0 : (i == n - 1 ? 2 : 1); }
 
-// A red-black cell pair (y = 2j, 2j + 1 of one row) as one thread keeps it:
-// cell 0 is the one that even phases update, cell 1 the other (the order of
-// the row's parity); Jacobi updates both in every phase. Addresses, right-
-// hand sides and 1/diag stay in registers over all phases, so an update is
-// four LDS reads, five FP64 operations and one LDS write. (Decoding the cell,
-// its boundary class and its neighbours in every phase instead was bound by
-// VALU issue: 26.7 us for a 128x32 tail, 6.7 us for a 256x64 tile launch.)
+// A cell pair (y = 2j, 2j + 1 of one row) as one thread keeps it: cell 0 is
+// the one that even red-black phases update, cell 1 the other (the order of
+// the row's parity); Jacobi updates both in every phase. Values, addresses,
+// right-hand sides and omega/diag stay in registers over all phases, and the
+// pair's cells are each other's neighbour, so an update is three LDS reads,
+// nine or ten operations and one LDS write. (Decoding the cell, its boundary
+// class and its neighbours in every phase instead was bound by VALU issue:
+// 26.7 us for a 128x32 tail, 6.7 us for a 256x64 tile launch.) A missing
+// neighbour's address is the cell's own: its difference is zero.
 template <class T>
 struct ChfPair {
-    int at[2], up, down;  // LDS elements; up and down belong to cell 0
-    T rhs[2], inv[2];
+    int at[2], outer[2], up, down;  // LDS elements; up and down belong to cell 0
+    T p[2], rhs[2], scale[2];       // scale: omega / diag
+    T outlet;                       // 2/hx^2 in the outlet row of a closed channel (value -p beyond it), else 0
 };
 
-template <class T>
-__device__ __forceinline__ T chf_update(const T* a, int at, int up, int down, T rhs, T inv, T wx, T wy) {
-    return fma_of(wy, a[at + 1] + a[at - 1], fma_of(wx, a[up] + a[down], rhs)) * inv;
+// The new value of cell o from the iterate `a`.
+template <class T, bool P>
+__device__ __forceinline__ T chf_update(const T* a, const ChfPair<T>& c, int o, T wx, T wy) {
+    const int step = c.at[o] - c.at[0];
+    const T p = c.p[o], dx = (a[c.up + step] - p) + (a[c.down + step] - p), dy = (a[c.outer[o]] - p) + (c.p[1 - o] - p);
+    T r = fma_of(wy, dy, fma_of(wx, dx, c.rhs[o]));
+    if (!P) r = fma_of(-c.outlet, p, r);
+    return fma_of(c.scale[o], r, p);
 }
 
 // One launch's share of level l: tile `tile` of chunk `chunk` of the pre-
@@ -156,36 +166,43 @@ __device__ __forceinline__ void chf_tile(const afsi_mg2d_plan& pl, int l, int ti
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int o = lead ^ s;
+            const bool wall = o ? gy + 2 == d.ny : gy == 0;
             c[q].at[s] = held ? at + o : CHF_PITCH + 1;
+            c[q].outer[s] = c[q].at[s] + (wall ? 0 : (o ? 1 : -1));
+            c[q].p[s] = o ? v[1] : v[0];
             c[q].rhs[s] = o ? b[1] : b[0];
             depth[q][s] = inside ? min(across, min(j + o, span - 1 - j - o)) : 0;
         }
-        c[q].up = c[q].at[0] + CHF_PITCH;
-        c[q].down = c[q].at[0] - CHF_PITCH;
+        c[q].up = c[q].at[0] + (P || gx + 1 != d.nx ? CHF_PITCH : 0);
+        c[q].down = c[q].at[0] - (P || gx != 0 ? CHF_PITCH : 0);
+        c[q].outlet = !P && gx + 1 == d.nx ? T(2) * k.ihx2 : T(0);
     }
+    const T omega = gs ? T(1) : T(pl.omega);
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < ROWS; ++q)
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int y = gy + ((row[q] & 1) ^ s), cx = P ? 1 : chf_class(row[q], d.nx);
-            c[q].inv[s] = row[q] >= 0 ? tab[3 * cx + chf_class(y, d.ny)] : T(0);
+            c[q].scale[s] = row[q] >= 0 ? omega * tab[3 * cx + chf_class(y, d.ny)] : T(0);
         }
 
     T* a = box;
     T* w = gs ? box : box + SIZE;
-    const T omega = T(pl.omega);
     for (int s = 0; s < count; ++s) {
         const int mine = (first + s) & 1;
 #pragma unroll
-        for (int q = 0; q < ROWS; ++q)
+        for (int q = 0; q < ROWS; ++q) {
+            T v[2] = {c[q].p[0], c[q].p[1]};
 #pragma unroll
             for (int o = 0; o < 2; ++o) {
                 if ((gs && o != mine) || depth[q][o] <= s) continue;
-                const int at = c[q].at[o], step = at - c[q].at[0];
-                const T v = chf_update(a, at, c[q].up + step, c[q].down + step, c[q].rhs[o], c[q].inv[o], k.ihx2, k.ihy2);
-                w[at] = gs ? v : a[at] + omega * (v - a[at]);
+                v[o] = chf_update<T, P>(a, c[q], o, k.ihx2, k.ihy2);
+                w[c[q].at[o]] = v[o];
             }
+            c[q].p[0] = v[0];
+            c[q].p[1] = v[1];
+        }
         __syncthreads();
         T* t = a; a = w; w = t;
     }
@@ -223,11 +240,11 @@ __device__ __forceinline__ void chf_tile(const afsi_mg2d_plan& pl, int l, int ti
 }
 
 // ---- the lower levels in one workgroup ---------------------------------------
-// LDS of level l: p as rows of ny + 2 cells (zero at the walls) and one more
-// row of zeros (the neighbour of a missing neighbour), a second p for Jacobi,
-// and rhs. The coarsest level keeps p and rhs without ghosts.
+// LDS of level l: p as rows of ny + 2 words (an even pitch other than ny, a
+// power of two as a rule, spreads rows over the banks), a second p for Jacobi,
+// and rhs. The coarsest level keeps p and rhs in cell order.
 __host__ __device__ inline int chf_box_cells(const afsi_mg2d_plan& pl, int l) {
-    return int((pl.n[l][0] + 1) * (pl.n[l][1] + 2));
+    return int(pl.n[l][0] * (pl.n[l][1] + 2));
 }
 
 __host__ __device__ inline int chf_level_values(const afsi_mg2d_plan& pl, int l) {
@@ -276,6 +293,7 @@ template <class T, bool P>
 __device__ __forceinline__ void chf_smooth(const ChfLevel<T> v, bool gs, int phases, T omega, T* lds, const T* tab) {
     const ChfPairs pairs(v.nx, v.ny);
     const int pitch = v.ny + 2;
+    T *a = lds + v.p, *w = gs ? a : lds + v.q;
     ChfPair<T> c[CHF_TAIL_PAIRS];
 #pragma unroll
     for (int q = 0; q < CHF_TAIL_PAIRS; ++q) {
@@ -283,35 +301,38 @@ __device__ __forceinline__ void chf_smooth(const ChfLevel<T> v, bool gs, int pha
         if (e >= pairs.n) continue;
         int x, j;
         pairs.at(e, x, j);
-        const int missing = v.nx * pitch;  // the row of zeros
-        const int above = x + 1 < v.nx ? (x + 1) * pitch : (P ? 0 : missing);
-        const int below = x > 0 ? (x - 1) * pitch : (P ? (v.nx - 1) * pitch : missing);
+        const int above = (x + 1 < v.nx ? x + 1 : (P ? 0 : x)) * pitch;
+        const int below = (x > 0 ? x - 1 : (P ? v.nx - 1 : x)) * pitch;
         const int lead = x & 1, cx = P ? 1 : chf_class(x, v.nx);
         const T* r = lds + v.r + x * v.ny + 2 * j;
         const T r0 = r[0], r1 = r[1];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const int y = 2 * j + (lead ^ s);
+            const int o = lead ^ s, y = 2 * j + o, outer = o ? y + 1 : y - 1;
             c[q].at[s] = x * pitch + y + 1;
-            c[q].inv[s] = tab[3 * cx + chf_class(y, v.ny)];
-            c[q].rhs[s] = (lead ^ s) ? r1 : r0;
+            c[q].outer[s] = x * pitch + (outer < 0 || outer == v.ny ? y : outer) + 1;
+            c[q].p[s] = a[c[q].at[s]];
+            c[q].scale[s] = omega * tab[3 * cx + chf_class(y, v.ny)];
+            c[q].rhs[s] = o ? r1 : r0;
         }
+        c[q].outlet = !P && x + 1 == v.nx ? T(2) * v.wx : T(0);
         c[q].up = above + 2 * j + lead + 1;
         c[q].down = below + 2 * j + lead + 1;
     }
-    T *a = lds + v.p, *w = gs ? a : lds + v.q;
     for (int s = 0; s < phases; ++s) {
         const int mine = s & 1;
 #pragma unroll
         for (int q = 0; q < CHF_TAIL_PAIRS; ++q) {
             if (int(threadIdx.x) + q * CHF_TAIL_NT >= pairs.n) continue;
+            T u[2] = {c[q].p[0], c[q].p[1]};
 #pragma unroll
             for (int o = 0; o < 2; ++o) {
                 if (gs && o != mine) continue;
-                const int at = c[q].at[o], step = at - c[q].at[0];
-                const T u = chf_update(a, at, c[q].up + step, c[q].down + step, c[q].rhs[o], c[q].inv[o], v.wx, v.wy);
-                w[at] = gs ? u : a[at] + omega * (u - a[at]);
+                u[o] = chf_update<T, P>(a, c[q], o, v.wx, v.wy);
+                w[c[q].at[o]] = u[o];
             }
+            c[q].p[0] = u[0];
+            c[q].p[1] = u[1];
         }
         __syncthreads();
         T* t = a; a = w; w = t;
@@ -321,7 +342,7 @@ __device__ __forceinline__ void chf_smooth(const ChfLevel<T> v, bool gs, int pha
         for (int q = 0; q < CHF_TAIL_PAIRS; ++q)
             if (int(threadIdx.x) + q * CHF_TAIL_NT < pairs.n)
 #pragma unroll
-                for (int o = 0; o < 2; ++o) w[c[q].at[o]] = a[c[q].at[o]];
+                for (int o = 0; o < 2; ++o) w[c[q].at[o]] = c[q].p[o];
         __syncthreads();
     }
 }
@@ -340,7 +361,7 @@ template <class T, bool P>
 __device__ __forceinline__ void chf_tail(const afsi_mg2d_plan& pl, int l0, int cycles, T* lds, ChfShared<T>& sh) {
     const int last = pl.levels - 1, tid = int(threadIdx.x), phases = chf_phases(pl);
     const bool gs = pl.smoother == 1;
-    const T omega = T(pl.omega);
+    const T omega = gs ? T(1) : T(pl.omega);
     int total = 0;
     for (int l = l0; l <= last; ++l) {
         const int cells = int(pl.n[l][0] * pl.n[l][1]), box = l == last ? cells : chf_box_cells(pl, l);

@@ -46,3 +46,37 @@ def test_one_level(gpu):
     ref = mac2d.ChannelMultigrid((9, 5), grid.spacing, OOptions(), False)
     want = ref.cycle(0, np.zeros((9, 5)), rhs)
     assert np.linalg.norm(got - want) < 1e-12 * np.linalg.norm(want)
+
+
+# Closed and periodic; the whole hierarchy in the tail, and one tiled level.
+@pytest.mark.parametrize('periodic', [False, True], ids=['closed', 'periodic'])
+@pytest.mark.parametrize('smoother,nu', [('rbgs', 2), ('jacobi', 4)])
+@pytest.mark.parametrize('shape', [(64, 16), (160, 32)])
+def test_cycles_stagnate_no_higher_than_the_oracle(gpu, shape, smoother, nu, periodic):
+    """Where V-cycles stop converging, the residual is what the rounding of the
+    stored iterate leaves (A applied to errors of half an ulp) plus that of one
+    update. The oracle updates in difference form, p + (rhs - A p) / diag,
+    whose own rounding is that of a small correction. Sums of the neighbours
+    themselves, (rhs + sum w p) / diag, stagnate 1.45 to 1.85 times higher. The
+    mean over five cycles varies by a few percent."""
+    grid = ChannelGrid(shape, (4., 1.3), periodic)
+    ref = mac2d.ChannelMultigrid(shape, grid.spacing, OOptions(smooth=nu, smoother=smoother), periodic)
+    rhs = np.random.default_rng(4).normal(size=shape)
+    if periodic:
+        rhs -= rhs.mean()
+    p, floor = np.zeros(shape), []
+    for i in range(25):
+        p = ref.cycle(0, p, rhs)
+        if i >= 20:
+            floor.append(np.linalg.norm(rhs - mac2d.negative_laplacian(p, grid.spacing, periodic)))
+    for dtype, unit in ((torch.float64, 1.), (torch.float32, 2. ** 29)):
+        mg = ChannelMultigrid(grid, device=gpu, dtype=dtype, options=MGOptions(smooth=nu, smoother=smoother),
+                              backend='workspace')
+        mg.p[0].zero_()
+        mg.rhs[0].copy_(torch.tensor(rhs))
+        got = []
+        for i in range(25):
+            mg.advance(1)
+            got.append(float(mg.results[0, 1].sqrt()))
+        print(shape, smoother, periodic, dtype, np.mean(got[20:]) / (np.mean(floor) * unit))
+        assert np.mean(got[20:]) <= 1.2 * np.mean(floor) * unit
