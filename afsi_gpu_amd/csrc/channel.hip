@@ -379,10 +379,16 @@ int ch_prolong(const T* coarse, T* fine, const int64_t n[2], int periodic, hipSt
 #include "channel_vcycle.hpp"
 
 template <class T>
-__global__ void __launch_bounds__(CHF_NT) chf_tile_kernel(afsi_mg2d_plan pl, int l, int chunk, bool up) {
+__global__ void __launch_bounds__(CHF_NT) chf_tile_kernel(afsi_mg2d_plan pl, int l, int chunk, bool up, int parts) {
     __shared__ T box[2 * CHF_B * CHF_PITCH], tab[9];
-    if (pl.periodic) chf_tile<T, true>(pl, l, int(blockIdx.x), chunk, up, box, tab);
-    else chf_tile<T, false>(pl, l, int(blockIdx.x), chunk, up, box, tab);
+    if (pl.periodic) {
+        // level 0 is restricted without the mean of rhs[0] (`parts` partials in the reduction scratch)
+        const bool removes = l == 0 && !up && chunk + 1 == chf_chunks(pl);
+        const T mean = removes ? T(chf_mean(pl.reduce_partials, parts, 4, int(pl.n[0][0] * pl.n[0][1]))) : T(0);
+        chf_tile<T, true>(pl, l, int(blockIdx.x), chunk, up, mean, box, tab);
+    } else {
+        chf_tile<T, false>(pl, l, int(blockIdx.x), chunk, up, T(0), box, tab);
+    }
 }
 
 template <class T, bool P>
@@ -396,11 +402,7 @@ __global__ void __launch_bounds__(CHF_TAIL_NT) chf_tail_kernel(afsi_mg2d_plan pl
 template <class T>
 __global__ void __launch_bounds__(CH_THREADS) ch_sub_partials_kernel(T* __restrict__ x, int count,
                                                                      const double* __restrict__ partials, int parts) {
-    double v = 0.0;
-    for (int b = int(threadIdx.x) % WAVE; b < parts; b += WAVE) v += partials[4 * b];
-#pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) v += __shfl_xor(v, dd, WAVE);
-    const T mean = T(v / double(count));
+    const T mean = T(chf_mean(partials, parts, 4, count));
     for (int i = blockIdx.x * CH_THREADS + threadIdx.x; i < count; i += gridDim.x * CH_THREADS) x[i] = x[i] - mean;
 }
 
@@ -497,9 +499,12 @@ static int channel_cycles(const afsi_mg2d_plan* pl, int32_t cycles, void* stream
     const int l0 = chf_split(*pl, sizeof(T), &bytes);
     if (l0 == 0) return channel_tail<T>(*pl, 0, cycles, bytes, s);
     const int chunks = chf_chunks(*pl);
+    const int64_t count = pl->n[0][0] * pl->n[0][1], parts = afsi_reduce_partials(count);
+    if (pl->periodic)
+        if (int r = launch_reduce_partials(static_cast<const T*>(pl->rhs[0]), count, pl->reduce_partials, s)) return r;
     const auto level = [&](int l, bool up) {
         for (int c = 0; c < chunks; ++c)
-            chf_tile_kernel<T><<<unsigned(chf_tiles(*pl, l)), CHF_NT, 0, s>>>(*pl, l, c, up);
+            chf_tile_kernel<T><<<unsigned(chf_tiles(*pl, l)), CHF_NT, 0, s>>>(*pl, l, c, up, int(parts));
     };
     for (int c = 0; c < cycles; ++c) {
         for (int l = 0; l < l0; ++l) level(l, false);
@@ -508,9 +513,8 @@ static int channel_cycles(const afsi_mg2d_plan* pl, int32_t cycles, void* stream
         AFSI_LAUNCH_CHECK();
     }
     if (!pl->periodic) return OK;
-    const int64_t count = pl->n[0][0] * pl->n[0][1], parts = afsi_reduce_partials(count);
     T* p = static_cast<T*>(pl->p[0]);
-    if (int r = launch_reduce_partials(p, count, pl->reduce_partials, s)) return r;
+    if (int r = launch_reduce_partials<T>(p, count, pl->reduce_partials, s)) return r;
     ch_sub_partials_kernel<T><<<grid_for(count, CH_THREADS, 1024), CH_THREADS, 0, s>>>(p, int(count),
                                                                                      pl->reduce_partials, int(parts));
     AFSI_LAUNCH_CHECK();
@@ -986,6 +990,9 @@ __global__ void __launch_bounds__(CH_THREADS) chb_correct_kernel(const ChbDesc* 
 // The launches of channel_cycles over every instance that has the level: a
 // work list per level holds the instances with their first tile, and the
 // tails run one workgroup per instance.
+constexpr int MLB_THREADS = 256;
+constexpr int MLB_CHUNK = 2048;  // level-0 cells per workgroup of the reductions
+
 struct MlbEntry {
     int32_t inst, block_begin;
 };
@@ -1003,14 +1010,24 @@ __device__ inline MlbEntry mlb_find(const MlbEntry* __restrict__ list, int n) {
 __global__ void __launch_bounds__(CHF_NT) chf_tile_batch_kernel(const afsi_mg2d_plan* __restrict__ plans,
                                                                 const MlbEntry* __restrict__ list, int n, int l,
                                                                 int chunk, bool up,
-                                                                const int32_t* __restrict__ active) {
+                                                                const int32_t* __restrict__ active,
+                                                                const MlbEntry* __restrict__ sums,
+                                                                const double* __restrict__ partials) {
     __shared__ double box[2 * CHF_B * CHF_PITCH], tab[9];
     const MlbEntry e = mlb_find(list, n);
     const afsi_mg2d_plan& pl = plans[e.inst];
     if ((active && !active[e.inst]) || chunk >= chf_chunks(pl)) return;
     const int tile = int(blockIdx.x) - e.block_begin;
-    if (pl.periodic) chf_tile<double, true>(pl, l, tile, chunk, up, box, tab);
-    else chf_tile<double, false>(pl, l, tile, chunk, up, box, tab);
+    if (pl.periodic) {
+        double mean = 0.0;
+        if (l == 0 && !up && chunk + 1 == chf_chunks(pl)) {  // the instance's partial sums of rhs[0]
+            const int count = int(pl.n[0][0] * pl.n[0][1]);
+            mean = chf_mean(partials + sums[e.inst].block_begin, (count + MLB_CHUNK - 1) / MLB_CHUNK, 1, count);
+        }
+        chf_tile<double, true>(pl, l, tile, chunk, up, mean, box, tab);
+    } else {
+        chf_tile<double, false>(pl, l, tile, chunk, up, 0.0, box, tab);
+    }
 }
 
 // Tails of the instances of one boundary type: those that start at level 0
@@ -1028,21 +1045,19 @@ __global__ void __launch_bounds__(CHF_TAIL_NT) chf_tail_batch_kernel(const afsi_
     chf_tail<double, P>(pl, l0, cycles, reinterpret_cast<double*>(raw), sh);
 }
 
-constexpr int MLB_THREADS = 256;
-constexpr int MLB_CHUNK = 2048;  // level-0 cells per workgroup of the reductions
-
-// Mean removal of p[0] after the cycles of periodic instances whose level 0
-// is tiled: partial sums per chunk, then the instance's partials in chunk order.
+// Sums of rhs[0] (before the cycles) or p[0] (after them, to remove its mean)
+// of periodic instances whose level 0 is tiled: partial sums per chunk, which
+// chf_mean adds.
 __global__ void __launch_bounds__(MLB_THREADS) mlb_sum_kernel(const afsi_mg2d_plan* __restrict__ plans,
                                                               const MlbEntry* __restrict__ list, int n,
                                                               const int32_t* __restrict__ split,
-                                                              const int32_t* __restrict__ active,
+                                                              const int32_t* __restrict__ active, bool rhs,
                                                               double* __restrict__ partials) {
     __shared__ double red[MLB_THREADS / WAVE];
     const MlbEntry e = mlb_find(list, n);
     const afsi_mg2d_plan& pl = plans[e.inst];
     if ((active && !active[e.inst]) || !pl.periodic || split[e.inst] == 0) return;
-    const double* x = static_cast<const double*>(pl.p[0]);
+    const double* x = static_cast<const double*>(rhs ? pl.rhs[0] : pl.p[0]);
     const int count = int(pl.n[0][0] * pl.n[0][1]);
     const int begin = (int(blockIdx.x) - e.block_begin) * MLB_CHUNK, end = min(begin + MLB_CHUNK, count);
     double v = 0.0;
@@ -1069,11 +1084,7 @@ __global__ void __launch_bounds__(MLB_THREADS) mlb_sub_kernel(const afsi_mg2d_pl
     double* x = static_cast<double*>(pl.p[0]);
     const int count = int(pl.n[0][0] * pl.n[0][1]), blocks = (count + MLB_CHUNK - 1) / MLB_CHUNK;
     const int begin = (int(blockIdx.x) - e.block_begin) * MLB_CHUNK, end = min(begin + MLB_CHUNK, count);
-    double v = 0.0;
-    for (int b = int(threadIdx.x) % WAVE; b < blocks; b += WAVE) v += partials[e.block_begin + b];
-#pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) v += __shfl_xor(v, dd, WAVE);
-    const double mean = v / double(count);
+    const double mean = chf_mean(partials + e.block_begin, blocks, 1, count);
     for (int i = begin + int(threadIdx.x); i < end; i += MLB_THREADS) x[i] = x[i] - mean;
 }
 
@@ -1416,9 +1427,16 @@ int afsi_chb_cycles_f64(const afsi_chb_batch* batch, const int32_t* active, int3
     if (int r = tails(true, cycles)) return r;
     if (L.maxsplit == 0) return OK;
     const auto list = [&](int l) { return chb_at<MlbEntry>(batch, L.lists) + size_t(l) * L.n; };
+    double* partials = chb_at<double>(batch, L.partials);
+    const MlbEntry* sums = list(AFSI_MG_MAX_LEVELS);
+    const auto sum = [&](bool rhs) {
+        mlb_sum_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, sums, L.n, split, active, rhs, partials);
+    };
+    if (L.mean) sum(true);
     const auto level = [&](int l, bool up) {
         for (int c = 0; c < L.chunks[l]; ++c)
-            chf_tile_batch_kernel<<<unsigned(L.blocks[l]), CHF_NT, 0, s>>>(plans, list(l), L.count[l], l, c, up, active);
+            chf_tile_batch_kernel<<<unsigned(L.blocks[l]), CHF_NT, 0, s>>>(plans, list(l), L.count[l], l, c, up, active,
+                                                                          sums, partials);
     };
     for (int c = 0; c < cycles; ++c) {
         for (int l = 0; l < L.maxsplit; ++l) level(l, false);
@@ -1427,10 +1445,8 @@ int afsi_chb_cycles_f64(const afsi_chb_batch* batch, const int32_t* active, int3
         AFSI_LAUNCH_CHECK();
     }
     if (!L.mean) return OK;
-    double* partials = chb_at<double>(batch, L.partials);
-    const MlbEntry* chunks = list(AFSI_MG_MAX_LEVELS);
-    mlb_sum_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, chunks, L.n, split, active, partials);
-    mlb_sub_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, chunks, L.n, split, active, partials);
+    sum(false);
+    mlb_sub_kernel<<<unsigned(L.reduce_blocks), MLB_THREADS, 0, s>>>(plans, sums, L.n, split, active, partials);
     AFSI_LAUNCH_CHECK();
     return OK;
 }

@@ -21,10 +21,14 @@
 // (low end, interior, high end of each axis). Differences of neighbours are
 // nearly exact and the quotient is a small correction, so a stored value
 // carries little more than its own rounding; in the form (b + sum w nb) / diag
-// the residual stagnates 1.45 to 3 times higher. The periodic channel's means are not removed inside a
-// cycle: A 1 = 0, smoothing, restriction and prolongation commute with a
-// constant shift and the coarse inverse of a zero-mean residual has zero mean,
-// so the driver removes the mean of p once after the last cycle.
+// the residual stagnates 1.45 to 3 times higher.
+//
+// Means of a periodic channel: A p has mean zero, so every residual has the
+// mean of rhs[0], and so has its restriction. That mean is subtracted once, as
+// level 0 is restricted; what is left below is rounding, which the coarse
+// product drops (its inverse would return it as a shift of p). The mean of p
+// is removed after the last cycle only: A 1 = 0, and smoothing, restriction
+// and prolongation commute with a constant shift.
 
 constexpr int CHF_T = 16;                    // tile edge
 constexpr int CHF_MAX = 7;                   // phases per launch (halo CHF_MAX + 1 <= CHF_T / 2)
@@ -36,6 +40,16 @@ static_assert(CHF_B == 2 * CHF_T, "two rows and one pair of columns per thread")
 constexpr int CHF_TAIL_NT = 1024;
 constexpr size_t CHF_TAIL_LDS = 150 * 1024;  // of 160 KB; the tables and reductions take the rest
 constexpr int CHF_TAIL_PAIRS = 2;            // cell pairs per thread: levels of at most 4096 cells
+
+// Mean of `count` values from `parts` partial sums, `stride` apart, in every
+// lane and in a fixed order.
+__device__ inline double chf_mean(const double* __restrict__ partials, int parts, int stride, int count) {
+    double v = 0.0;
+    for (int b = int(threadIdx.x) % WAVE; b < parts; b += WAVE) v += partials[int64_t(b) * stride];
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) v += __shfl_xor(v, dd, WAVE);
+    return v / double(count);
+}
 
 // Phases of one smoothing stage.
 __host__ __device__ inline int chf_phases(const afsi_mg2d_plan& pl) { return pl.smoother == 1 ? 2 * pl.nu : pl.nu; }
@@ -97,9 +111,10 @@ __device__ __forceinline__ T chf_update(const T* a, const ChfPair<T>& c, int o, 
 // that chunk c - 1 wrote; p and tmp alternate, and both stages have the same
 // number of chunks, so the level's iterate ends in p. The halo is even, so a
 // thread's cell pairs are the children of coarse cells. A cell is updated in
-// phase s while it lies more than s cells from the box edge.
+// phase s while it lies more than s cells from the box edge. `mean` is
+// subtracted from the restricted residual.
 template <class T, bool P>
-__device__ __forceinline__ void chf_tile(const afsi_mg2d_plan& pl, int l, int tile, int chunk, bool up, T* box,
+__device__ __forceinline__ void chf_tile(const afsi_mg2d_plan& pl, int l, int tile, int chunk, bool up, T mean, T* box,
                                          T* tab) {
     const Dim2 d{int(pl.n[l][0]), int(pl.n[l][1])};
     const Coef2<T> k = chf_coef<T>(pl, l);
@@ -234,7 +249,7 @@ __device__ __forceinline__ void chf_tile(const afsi_mg2d_plan& pl, int l, int ti
             const T r10 = __shfl_down(r[0], CHF_T, WAVE), r11 = __shfl_down(r[1], CHF_T, WAVE);
             if (mine && !(i & 1))
                 static_cast<T*>(pl.rhs[l + 1])[(row[q] / 2) * (d.ny / 2) + gy / 2] =
-                    (((r[0] + r[1]) + r10) + r11) * T(0.25);
+                    (((r[0] + r[1]) + r10) + r11) * T(0.25) - mean;
         }
     }
 }
@@ -401,6 +416,24 @@ __device__ __forceinline__ void chf_tail(const afsi_mg2d_plan& pl, int l0, int c
         }
     }
     __syncthreads();
+    // mean of the n words at x (LDS), in every thread
+    const auto mean_of = [&](const T* x, int n, int pitch) -> T {
+        const float inverse = 1.0f / float(top.ny);
+        double sum = 0.0;
+        for (int i = tid; i < n; i += CHF_TAIL_NT) {
+            const int r = int((float(i) + 0.5f) * inverse);
+            sum += double(x[r * pitch + i - r * top.ny]);
+        }
+#pragma unroll
+        for (int dd = 32; dd >= 1; dd >>= 1) sum += __shfl_xor(sum, dd, WAVE);
+        if (lane == 0) sh.red[wave] = sum;
+        __syncthreads();
+        sum = 0.0;
+        for (int w = 0; w < CHF_TAIL_NT / WAVE; ++w) sum += sh.red[w];
+        return T(sum / double(n));
+    };
+    const int cells = top.nx * top.ny;
+    const T rhs_mean = P && l0 == 0 && l0 < last ? mean_of(lds + top.r, cells, top.ny) : T(0);
     for (int cycle = 0; cycle < cycles; ++cycle) {
         for (int l = l0; l < last; ++l) {
             const ChfLevel<T> v = sh.level[l], c = sh.level[l + 1];
@@ -422,14 +455,20 @@ __device__ __forceinline__ void chf_tail(const afsi_mg2d_plan& pl, int l0, int c
                     if (!P && x == v.nx - 1) s += T(2) * v.wx * *f;
                     res[q] = lds[v.r + x * v.ny + y] - s;
                 }
-                lds[c.r + e] = (((res[0] + res[1]) + res[2]) + res[3]) * T(0.25);
+                lds[c.r + e] = (((res[0] + res[1]) + res[2]) + res[3]) * T(0.25) - (l == 0 ? rhs_mean : T(0));
                 if (l + 1 < last) lds[c.p + X * (c.ny + 2) + Y + 1] = T(0);
             }
             __syncthreads();
         }
         const ChfLevel<T> bottom = sh.level[last];
         if (m <= WAVE) {
-            const T x = lane < m ? lds[bottom.r + lane] : T(0);
+            T x = lane < m ? lds[bottom.r + lane] : T(0);
+            if (P) {
+                T sum = x;
+#pragma unroll
+                for (int dd = 32; dd >= 1; dd >>= 1) sum += __shfl_xor(sum, dd, WAVE);
+                x = lane < m ? x - sum / T(m) : T(0);
+            }
 #pragma unroll
             for (int i = 0; i < ROWS; ++i) {
                 T acc = held[i] * x;
@@ -438,9 +477,16 @@ __device__ __forceinline__ void chf_tail(const afsi_mg2d_plan& pl, int l0, int c
                 if (lane == 0 && ROWS * wave + i < m) lds[bottom.p + ROWS * wave + i] = acc;
             }
         } else {
+            T mean = T(0);
+            if (P) {
+                for (int c = lane; c < m; c += WAVE) mean += lds[bottom.r + c];
+#pragma unroll
+                for (int dd = 32; dd >= 1; dd >>= 1) mean += __shfl_xor(mean, dd, WAVE);
+                mean /= T(m);
+            }
             for (int row = wave; row < m; row += CHF_TAIL_NT / WAVE) {
                 T acc = T(0);
-                for (int c = lane; c < m; c += WAVE) acc += A[row * m + c] * lds[bottom.r + c];
+                for (int c = lane; c < m; c += WAVE) acc += A[row * m + c] * (lds[bottom.r + c] - mean);
 #pragma unroll
                 for (int dd = 32; dd >= 1; dd >>= 1) acc += __shfl_xor(acc, dd, WAVE);
                 if (lane == 0) lds[bottom.p + row] = acc;
@@ -483,24 +529,10 @@ __device__ __forceinline__ void chf_tail(const afsi_mg2d_plan& pl, int l0, int c
             chf_smooth<T, P>(v, gs, phases, omega, lds, sh.tab[l]);
         }
     }
-    const int cells = top.nx * top.ny, pitch = l0 == last ? top.ny : top.ny + 2;
+    const int pitch = l0 == last ? top.ny : top.ny + 2;
     const T* src = lds + top.p + (l0 == last ? 0 : 1);
     const float inverse = 1.0f / float(top.ny);
-    T mean = T(0);
-    if (P && l0 == 0) {
-        double sum = 0.0;
-        for (int i = tid; i < cells; i += CHF_TAIL_NT) {
-            const int x = int((float(i) + 0.5f) * inverse), y = i - x * top.ny;
-            sum += double(src[x * pitch + y]);
-        }
-#pragma unroll
-        for (int dd = 32; dd >= 1; dd >>= 1) sum += __shfl_xor(sum, dd, WAVE);
-        if (lane == 0) sh.red[wave] = sum;
-        __syncthreads();
-        sum = 0.0;
-        for (int w = 0; w < CHF_TAIL_NT / WAVE; ++w) sum += sh.red[w];
-        mean = T(sum / double(cells));
-    }
+    const T mean = P && l0 == 0 ? mean_of(src, cells, pitch) : T(0);
     T* out = static_cast<T*>(pl.p[l0]);
     for (int i = tid; i < cells; i += CHF_TAIL_NT) {
         const int x = int((float(i) + 0.5f) * inverse), y = i - x * top.ny;

@@ -3,12 +3,16 @@ workgroup tail, the tiles' edges and the phase chunks can go wrong: levels on
 either side of the tail's capacity (128x32, 160x32), extents that are no
 multiple of the 16-cell tile, sweeps that need two launches per stage, and a
 hierarchy of one level; against the oracle's cycle."""
+from ctypes import byref
+
 import numpy as np
 import pytest
 import torch
 
+from afsi_gpu_amd import _abi
 from afsi_gpu_amd.mac import MGOptions
 from afsi_gpu_amd.mac2d import ChannelGrid, ChannelMultigrid
+from afsi_gpu_amd.mac2d.batch import BatchedChannelStep
 from oracle import mac2d
 from oracle.mac3d import MGOptions as OOptions
 
@@ -80,3 +84,29 @@ def test_cycles_stagnate_no_higher_than_the_oracle(gpu, shape, smoother, nu, per
             got.append(float(mg.results[0, 1].sqrt()))
         print(shape, smoother, periodic, dtype, np.mean(got[20:]) / (np.mean(floor) * unit))
         assert np.mean(got[20:]) <= 1.2 * np.mean(floor) * unit
+
+
+# whole hierarchy in the tail; one, two and three tiled levels; two launches per stage
+@pytest.mark.parametrize('shape,smoother,nu', [((64, 16), 'rbgs', 2), ((160, 32), 'rbgs', 2), ((512, 64), 'jacobi', 4),
+                                               ((512, 128), 'rbgs', 2), ((1024, 128), 'rbgs', 5), ((48, 20), 'jacobi', 3)])
+def test_periodic_cycle_of_a_rhs_with_a_mean(gpu, shape, smoother, nu):
+    """A periodic cycle's coarse problems have zero mean whatever the mean of the
+    right-hand side, singly and in a batch."""
+    grid = ChannelGrid(shape, (4., 1.3), True)
+    ref = mac2d.ChannelMultigrid(shape, grid.spacing, OOptions(smooth=nu, smoother=smoother), True)
+    gen = np.random.default_rng(12)
+    p, rhs = gen.normal(size=shape) + .7, gen.normal(size=shape) + 3.
+    want = ref.cycle(0, p, rhs)
+    for dtype, bound in ((torch.float64, 1e-12), (torch.float32, 1e-12 * 2. ** 29)):
+        mg = ChannelMultigrid(grid, device=gpu, dtype=dtype, options=MGOptions(smooth=nu, smoother=smoother),
+                              backend='workspace')
+        got = mg.cycle(torch.tensor(p, device=gpu, dtype=dtype), torch.tensor(rhs, device=gpu, dtype=dtype))
+        assert np.linalg.norm(got.double().cpu().numpy() - want) < bound * np.linalg.norm(want)
+    other = ChannelGrid((32, 16), (2., 1.), False)
+    batch = BatchedChannelStep([other, grid], [1, 1], dt=1e-3, device=gpu,
+                               options=MGOptions(smooth=nu, smoother=smoother))
+    solver = batch.solvers[1]
+    solver.p[0].copy_(torch.tensor(p))
+    solver.rhs[0].copy_(torch.tensor(rhs))
+    _abi.call('afsi_chb_cycles_f64', byref(batch.batch), None, 1, _abi.stream())
+    assert np.linalg.norm(solver.p[0].cpu().numpy() - want) < 1e-12 * np.linalg.norm(want)
