@@ -201,13 +201,35 @@ __device__ __forceinline__ void coarse_stage(const CoarseArgs<T>& a, int l, bool
             }
         }
     } else {
+        // difference form, p + omega (b - sum w (p - nb)) / diag, as on the
+        // tiled levels; a missing neighbour's place is the cell's own
+        int nb[COARSE_PAIRS][2][5];
+#pragma unroll
+        for (int q = 0; q < COARSE_PAIRS; ++q) {
+            const int e = tid + q * COARSE_THREADS;
+            if (e >= np) continue;
+#pragma unroll
+            for (int colour = 0; colour < 2; ++colour) {
+                const int from[5] = {xp[q], xm[q], yp[q], ym[q], zo[q][colour]};
+#pragma unroll
+                for (int i = 0; i < 5; ++i) nb[q][colour][i] = !P && from[i] == np ? e + (colour ? cs : -cs) : from[i];
+                inv[q][colour] *= a.omega;
+            }
+        }
         for (int it = 0; it < a.nu; ++it) {
             T w[COARSE_PAIRS][2];
 #pragma unroll
             for (int q = 0; q < COARSE_PAIRS; ++q) {
                 if (tid + q * COARSE_THREADS >= np) continue;
-                w[q][0] = value(q, 0);
-                w[q][1] = value(q, 1);
+#pragma unroll
+                for (int colour = 0; colour < 2; ++colour) {
+                    const T* o = red + (1 - colour) * cs;
+                    const int* at = nb[q][colour];
+                    const T c = p[q][colour], zs = (p[q][1 - colour] - c) + (o[at[4]] - c);
+                    const T ys = (o[at[2]] - c) + (o[at[3]] - c), xs = (o[at[0]] - c) + (o[at[1]] - c);
+                    const T d = fma_of(k.w[0], xs, fma_of(k.w[1], ys, fma_of(k.w[2], zs, r[q][colour])));
+                    w[q][colour] = fma_of(inv[q][colour], d, c);
+                }
             }
             __syncthreads();
 #pragma unroll
@@ -215,7 +237,7 @@ __device__ __forceinline__ void coarse_stage(const CoarseArgs<T>& a, int l, bool
                 if (tid + q * COARSE_THREADS >= np) continue;
 #pragma unroll
                 for (int colour = 0; colour < 2; ++colour) {
-                    p[q][colour] += a.omega * (w[q][colour] - p[q][colour]);
+                    p[q][colour] = w[q][colour];
                     red[colour * cs + tid + q * COARSE_THREADS] = p[q][colour];
                 }
             }

@@ -13,6 +13,7 @@ from oracle import mac3d
 
 pytestmark = pytest.mark.gpu
 LENGTHS = (1., 1.3, .9)
+CYCLES = 60  # more than Jacobi cycles take to stagnate in FP64
 
 
 def check(gpu, shape, periodic, smoother, nu):
@@ -46,3 +47,34 @@ def test_cycle_matches_oracle(gpu, shape, smoother, nu, periodic):
 @pytest.mark.parametrize('smoother,nu', [('rbgs', 2), ('jacobi', 3)])
 def test_two_phase_level_matches_oracle(gpu, smoother, nu, periodic):
     check(gpu, (128, 80, 112), periodic, smoother, nu)
+
+
+@pytest.mark.parametrize('periodic', [False, True], ids=['closed', 'periodic'])
+@pytest.mark.parametrize('shape', [(16, 16, 16), (32, 24, 40)])
+def test_jacobi_stagnates_no_higher_than_the_oracle(gpu, shape, periodic):
+    """Where Jacobi cycles stop converging (the coarse kernel alone; tiled levels
+    above it), the residual is what the rounding of the stored iterate leaves
+    plus that of one update. The oracle's update p + omega (rhs - A p) / diag
+    rounds a small correction; (rhs + sum w p) / diag would stagnate 1.6 to 1.8
+    times higher. The mean over five cycles varies by a few percent."""
+    h = tuple(L / n for L, n in zip(LENGTHS, shape))
+    options = dict(smooth=4, smoother='jacobi')
+    ref = mac3d.Multigrid(shape, h, mac3d.MGOptions(**options), periodic)
+    rhs = np.random.default_rng(6).normal(size=shape)
+    rhs -= rhs.mean()
+    p, floor = np.zeros(shape), []
+    for i in range(CYCLES):
+        p = ref.cycle(0, p, rhs)
+        if i >= CYCLES - 5:
+            floor.append(np.linalg.norm(rhs - mac3d.negative_laplacian(p, h, periodic)))
+    assert floor[-1] > .5 * floor[0]  # stagnated
+    for dtype, unit in ((torch.float64, 1.), (torch.float32, 2. ** 29)):
+        mg = GeometricMultigrid(MACGrid(shape, LENGTHS, periodic=periodic), device=gpu, dtype=dtype,
+                                options=MGOptions(**options), backend='workspace')
+        mg.initialize(torch.zeros(shape, device=gpu, dtype=dtype), torch.tensor(rhs, device=gpu, dtype=dtype))
+        got = []
+        for i in range(CYCLES):
+            mg.advance(1)
+            got.append(float(mg.results[0, 1].sqrt()))
+        print(shape, periodic, dtype, np.mean(got[-5:]) / (np.mean(floor) * unit))
+        assert np.mean(got[-5:]) <= 1.2 * np.mean(floor) * unit
