@@ -184,8 +184,8 @@ __device__ __forceinline__ void coarse_stage(const CoarseArgs<T>& a, int l, bool
     __syncthreads();
     const auto value = [&](int q, int colour) -> T {
         const T* o = red + (1 - colour) * cs;
-        return gs_value<T>(k, r[q][colour], p[q][1 - colour] + o[zo[q][colour]], o[yp[q]] + o[ym[q]], o[xp[q]] + o[xm[q]],
-                           inv[q][colour]);
+        return gs_sum<T>(k, r[q][colour], p[q][1 - colour] + o[zo[q][colour]], o[yp[q]] + o[ym[q]], o[xp[q]] + o[xm[q]]) *
+               inv[q][colour];
     };
     if (a.smoother == 1) {
         for (int it = 0; it < a.nu; ++it) {

@@ -349,14 +349,27 @@ constexpr int ZROW = 128;
 
 __device__ inline int face_class(int g, int n) { return g == 0 ? 0 : (g == n - 1 ? 2 : 1); }
 
-// 1/diag of the Neumann operator by boundary class (0 low, 1 interior,
+// Diagonal of the Neumann operator by boundary class (0 low, 1 interior,
 // 2 high) per axis; entry t of a 27-table.
 template <class T>
-__device__ inline T inv_diag_entry(int t, const W3<T>& k) {
+__device__ inline T diag_entry(int t, const W3<T>& k) {
     const int cls[3] = {t / 9, (t / 3) % 3, t % 3};
     T dg = T(0);
     for (int a = 0; a < 3; ++a) dg += k.w[a] * T(cls[a] == 1 ? 2 : 1);
-    return T(1) / dg;
+    return dg;
+}
+template <class T>
+__device__ inline T inv_diag_entry(int t, const W3<T>& k) { return T(1) / diag_entry<T>(t, k); }
+
+// A reciprocal and what its rounding left out: t * hi + t * lo rounds like t / diag.
+template <class T>
+struct Recip {
+    T hi, lo;
+};
+template <class T>
+__device__ inline Recip<T> recip(T diag) {
+    const T r = T(1) / diag;
+    return {r, fma_of(-diag, r, T(1)) * r};
 }
 
 template <class T, bool P>
@@ -472,7 +485,7 @@ __device__ __forceinline__ void rb_rows_tiles(const T* __restrict__ pin, const T
     if (!P && threadIdx.x < 27) tab[threadIdx.x] = inv_diag_entry<T>(threadIdx.x, k);
     __syncthreads();
     fetch(0, first);
-    const T inv_p = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
+    const Recip<T> inv_p = recip(T(2) * (k.w[0] + k.w[1] + k.w[2]));
     auto update = [&](const T* row, int r, int gx, int gy, int z, T b) -> T {
         // a missing neighbour adds zero
         const T zs = (P || z + 1 < n2 ? row[P && z + 1 == n2 ? 0 : z + 1] : T(0)) +
@@ -480,7 +493,7 @@ __device__ __forceinline__ void rb_rows_tiles(const T* __restrict__ pin, const T
         const T ys = (P || gy + 1 < d.n1 ? box[(r + 1) * n2 + z] : T(0)) + (P || gy > 0 ? box[(r - 1) * n2 + z] : T(0));
         const T xs = (P || gx + 1 < d.n0 ? box[(r + BYr) * n2 + z] : T(0)) +
                      (P || gx > 0 ? box[(r - BYr) * n2 + z] : T(0));
-        const T inv = P ? inv_p : tab[face_class(gx, d.n0) * 9 + face_class(gy, d.n1) * 3 + face_class(z, n2)];
+        const Recip<T> inv = P ? inv_p : Recip<T>{tab[face_class(gx, d.n0) * 9 + face_class(gy, d.n1) * 3 + face_class(z, n2)], T(0)};
         return rb_relax(k, row[z], gs_value<T>(k, b, zs, ys, xs, inv));
     };
     for (int j = 0; j < count; ++j) {

@@ -71,12 +71,23 @@ __device__ inline int wrap_near(int g, int n) {
     return g;
 }
 
-// Gauss-Seidel value of a cell from the sums of its z, y and x neighbours;
-// every red-black kernel of the fused driver forms it this way, so they agree
-// bit for bit.
+// Gauss-Seidel value of a cell times its diagonal, from the sums of its z, y
+// and x neighbours.
 template <class T>
-__device__ __forceinline__ T gs_value(const W3<T>& k, T b, T zs, T ys, T xs, T inv) {
-    return (b + fma_of(k.w[0], xs, fma_of(k.w[1], ys, k.w[2] * zs))) * inv;
+__device__ __forceinline__ T gs_sum(const W3<T>& k, T b, T zs, T ys, T xs) {
+    return fma_of(k.w[0], xs, fma_of(k.w[1], ys, fma_of(k.w[2], zs, b)));
+}
+
+// The value. The row sweeps form it this way too, so they and the stages agree
+// bit for bit. A plain product with the rounded reciprocal (lo = 0) lets the
+// residual stagnate 1.1 to 1.2 times higher. Periodic levels have one
+// reciprocal, and lo costs nothing there. On closed levels its selects cost 3
+// to 11% of a cycle, so it is used only where the sweeps divide (z > ZROW), in
+// tiles away from the ends of x, which need no selects.
+template <class T>
+__device__ __forceinline__ T gs_value(const W3<T>& k, T b, T zs, T ys, T xs, const Recip<T>& inv) {
+    const T t = gs_sum(k, b, zs, ys, xs);
+    return fma_of(t, inv.hi, t * inv.lo);
 }
 
 template <class T, bool P, bool GS, int TX, int TY, int NPH, bool RESTRICT>
@@ -199,21 +210,25 @@ __device__ __forceinline__ void stage_tile(const StageArgs<T>& a, int tile, T* l
             r[(2 * i + 1) * G::TC] = RB[H + i];
         }
     }
+    const bool plain = P || (x0 > 0 && x0 + BX < d.n0);  // no plane at or beyond an end
     // 1/diag of red on even planes (= black on odd ones) and the other way
     // round, for planes inside (mid) and at the ends (end) of a closed domain
-    T mid[2], end[2];
+    T mid[2], end[2], lo[2];
     if (P) {
-        mid[0] = mid[1] = end[0] = end[1] = T(1) / (T(2) * (k.w[0] + k.w[1] + k.w[2]));
+        const Recip<T> r = recip(T(2) * (k.w[0] + k.w[1] + k.w[2]));
+        mid[0] = mid[1] = end[0] = end[1] = r.hi;
+        lo[0] = lo[1] = r.lo;
     } else {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int z = gz + (q ^ s);
             const int c = 3 * face_class(gy, d.n1) + face_class(z, d.n2);
-            mid[s] = inside ? inv_diag_entry<T>(9 + c, k) : T(0);
+            const Recip<T> m = recip(diag_entry<T>(9 + c, k));
+            mid[s] = inside ? m.hi : T(0);
             end[s] = inside ? inv_diag_entry<T>(c, k) : T(0);
+            lo[s] = inside && plain && d.n2 > ZROW ? m.lo : T(0);
         }
     }
-    const bool plain = P || (x0 > 0 && x0 + BX < d.n0);  // no plane at or beyond an end
     __syncthreads();
 
     const auto inverse = [&](int x, int s) -> T {
@@ -232,7 +247,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs<T>& a, int tile, T* l
             const T* z = (s ? zB : zA) + x * PL + (colour ? 0 : COLS);
             const T inner = colour ? A[x] : B[x];
             const T xs = colour ? A[x + 1] + A[x - 1] : B[x + 1] + B[x - 1];
-            return gs_value<T>(k, colour ? RB[x] : RA[x], inner + *z, o[HB] + o[-HB], xs, inverse(x, s));
+            return gs_value<T>(k, colour ? RB[x] : RA[x], inner + *z, o[HB] + o[-HB], xs,
+                               Recip<T>{inverse(x, s), lo[s]});
         };
 #pragma unroll
         for (int s = 0; s < NPH; ++s) {
