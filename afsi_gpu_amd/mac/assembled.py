@@ -167,7 +167,7 @@ class AssembledTransfer(FETransfer):
 
     def _rows(self, base, phi):
         """The three components by rows, or None where a row's stencil box
-        does not fit (the hash table takes those)."""
+        does not fit or there are no entries (the hash table takes those)."""
         g, A = self.geometry, self.geometry.cells.shape[1]
         (E, Q), N = g.weights.shape, g.node_count
         shapes = [self.grid.face_shape(c) for c in range(3)]
@@ -201,7 +201,8 @@ class AssembledTransfer(FETransfer):
         if flag:
             raise FloatingPointError('invalid hash IB entries: nonfinite values')
         nnz = ends[2]
-        if nnz >= 2 ** 31:  # the entries of all components are sorted together
+        # nothing to sort; or too much: the entries of all components are sorted together
+        if not 0 < nnz < 2 ** 31:
             return None
         row_ptr, b_cols, b_vals = empty(3, N + 1), empty(nnz), empty(nnz, dtype=torch.float64)
         face_ptr, t_cols, t_vals = empty(sum(faces) + 3), empty(nnz), empty(nnz, dtype=torch.float64)

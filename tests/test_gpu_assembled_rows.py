@@ -76,3 +76,13 @@ def test_rows_refuse_what_the_table_refused(gpu):
     stencil.base[2, 5, 0] = -1
     with pytest.raises(ValueError, match='stencil box'):
         tr._rows(stencil.base, stencil.phi)
+
+
+def test_operator_without_entries(gpu):
+    """Weights of zero leave no entries: preparing succeeds, as through the table."""
+    geometry, x = geometry_of('solid', gpu)
+    tr = AssembledTransfer(MACGrid((16, 18, 20), (1., 1., 1.)), geometry)
+    geometry.weights.zero_()
+    st = tr.prepare(x)
+    assert st.assembly['total_nnz'] == 0
+    assert all(int(m.row_ptr[-1]) == 0 and m.row_ptr.numel() == m.rows + 1 for m in st.gather + st.spread)
