@@ -36,7 +36,9 @@ namespace {
 constexpr int PT_STRIDE = 13;     // 12 phi + W N per point; odd: rows spread over the banks
 constexpr uint32_t ZERO_POINT = WAVE;  // a row of zeros after the points
 constexpr int CELL_WAVES = 4;
-constexpr int UNROLL = 4;              // chunks whose operands are read together
+constexpr int UNROLL = 4;              // chunks whose operands are read together; divides WAVE
+// Chunk slots per cell: a cell of Q points has at most Q chunks.
+__host__ __device__ inline int chunk_slots(int quad) { return (quad + UNROLL - 1) / UNROLL * UNROLL; }
 // What LDS holds: 128 KB of sites + 6.6 KB of points. Rows beat the table
 // wherever they fit: 0.28 / 2.78 ms for 468 nodes with rows up to 1320
 // sites, 0.34 / 5.12 ms up to 3808, 0.65 / 7.23 ms up to about 12000.
@@ -59,8 +61,8 @@ __device__ inline int wave_all(int v, Op op) {
 // points of each base in chunks of at most four: x = four point numbers of 8
 // bits, ZERO_POINT where there is none; y = the base relative to the box (8
 // bits per axis), and in the first chunk's top byte the number of chunks less
-// one. Groups by first appearance, points ascending; the list is filled to 64
-// with empty chunks.
+// one. Groups by first appearance, points ascending; the list is filled with
+// empty chunks.
 __global__ void __launch_bounds__(CELL_WAVES* WAVE) cell_order_kernel(afsi_fe_geometry g,
                                                                       const int64_t* __restrict__ base,
                                                                       afsi_grid3 grid, uint2* __restrict__ chunks,
@@ -69,7 +71,7 @@ __global__ void __launch_bounds__(CELL_WAVES* WAVE) cell_order_kernel(afsi_fe_ge
     __shared__ unsigned long long part[CELL_WAVES];
     __shared__ uint32_t ids[CELL_WAVES][WAVE], offs[CELL_WAVES][WAVE];
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, c = blockIdx.y;
-    const int Q = g.quad, A = g.nodes_per_cell;
+    const int Q = g.quad, A = g.nodes_per_cell, slots = chunk_slots(Q);
     const int64_t P = g.elements * Q;
     int64_t extent[3];
 #pragma unroll
@@ -138,7 +140,7 @@ __global__ void __launch_bounds__(CELL_WAVES* WAVE) cell_order_kernel(afsi_fe_ge
         __builtin_amdgcn_wave_barrier();
         uint2 chunk = make_uint2(ids[wave][lane], offs[wave][lane]);
         if (lane == 0) chunk.y |= uint32_t(start / 4 - 1) << 24;
-        chunks[(int64_t(c) * g.elements + e) * WAVE + lane] = chunk;
+        if (lane < slots) chunks[(int64_t(c) * g.elements + e) * slots + lane] = chunk;
         __builtin_amdgcn_wave_barrier();
     }
     if (lane == 0) part[wave] = raw;
@@ -202,7 +204,7 @@ __global__ void __launch_bounds__(WAVE) rows_kernel(afsi_fe_geometry g, const do
     const int64_t rows = 3 * g.node_count;
     const int64_t r = row_of_block(rows);
     if (blockIdx.x / 8 >= (rows + 7) / 8 || r >= rows) return;
-    const int lane = threadIdx.x, Q = g.quad, A = g.nodes_per_cell;
+    const int lane = threadIdx.x, Q = g.quad, A = g.nodes_per_cell, slots = chunk_slots(Q);
     const int64_t c = r / g.node_count, node = r - c * g.node_count;
     const int64_t P = g.elements * Q;
     const int l0 = row_box[r * 6], l1 = row_box[r * 6 + 1], l2 = row_box[r * 6 + 2];
@@ -229,7 +231,7 @@ __global__ void __launch_bounds__(WAVE) rows_kernel(afsi_fe_geometry g, const do
     const auto fetch = [&](int it) {
         const int64_t e = it / A, first = c * P + e * Q;
         const int q = min(lane, Q - 1);
-        chunk = chunks[(c * g.elements + e) * WAVE + lane];
+        chunk = chunks[(c * g.elements + e) * slots + min(lane, slots - 1)];
 #pragma unroll
         for (int j = 0; j < 6; ++j) f[j] = taps[first * 6 + min(j * WAVE + lane, Q * 6 - 1)];
         weight = g.weights[e * Q + q];
@@ -265,7 +267,7 @@ __global__ void __launch_bounds__(WAVE) rows_kernel(afsi_fe_geometry g, const do
         // lane i: first site of chunk i
         const int corner_of = (int(here.y & 255u) * w1 + int(here.y >> 8 & 255u)) * w2 + int(here.y >> 16 & 255u);
         const int n = int(__builtin_amdgcn_readlane(here.y, 0) >> 24) + 1;
-        for (int i = 0; i < n; i += UNROLL) {  // 64 is a multiple; the rest of a list is empty chunks
+        for (int i = 0; i < n; i += UNROLL) {  // the slots are a multiple; the rest of a list is empty chunks
             double u[UNROLL], v[UNROLL];
 #pragma unroll
             for (int j = 0; j < UNROLL; ++j) {

@@ -177,7 +177,8 @@ class AssembledTransfer(FETransfer):
             return None
         grid, device = self.grid.abi(), g.weights.device
         empty = lambda *shape, dtype=torch.int32: torch.empty(shape, dtype=dtype, device=device)
-        chunks, cell_box, row_box = empty(3, E, 64, dtype=torch.int64), empty(3, E, 6), empty(3 * N, 6)
+        slots = (Q + 3) // 4 * 4  # a cell's points in at most Q chunks
+        chunks, cell_box, row_box = empty(3, E, slots, dtype=torch.int64), empty(3, E, 6), empty(3 * N, 6)
         sites, counts = empty(3 * N, dtype=torch.int64), empty(3 * N, dtype=torch.int64)
         stats = torch.zeros(5, dtype=torch.int64, device=device)
         _abi.call('afsi_p1_row_boxes_f64', self._g, _abi.ptr(base), grid, _abi.ptr(chunks), _abi.ptr(cell_box),

@@ -784,8 +784,9 @@ int afsi_p1_contract_f64(const afsi_fe_geometry* g, const int64_t* base, const d
                          void* stream);
 /* The same operator for all three components at once, by rows: no table, no
  * order-dependent sums. Cells of at most 4 nodes and 64 points, closed boxes.
- * Step 1, boxes: chunks (3,E,64) uint64 lists each cell's points by
- * stencil base, four to a chunk, cell_box (3,E,6) and row_box (3*nodes,6) are stencil boxes, sites
+ * Step 1, boxes: chunks (3,E,S) uint64, S = points per cell rounded up to a
+ * multiple of four, lists each cell's points by stencil base, four to a
+ * chunk, cell_box (3,E,6) and row_box (3*nodes,6) are stencil boxes, sites
  * (3*nodes) the rows' box sizes. stats (5) int64, zero on entry: box sites of
  * all cells per component, largest row box if it exceeds 512, flag (1: a
  * cell's bases span more than 256 faces, 2: invalid cell table or stencil

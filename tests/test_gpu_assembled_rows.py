@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import fe as ofe
-from afsi_gpu_amd import workloads
+from afsi_gpu_amd import _abi, workloads
 from afsi_gpu_amd.mac.assembled import AssembledTransfer
 from afsi_gpu_amd.mac.fe import FEGeometry
 from afsi_gpu_amd.mac.grid import MACGrid
@@ -86,3 +86,33 @@ def test_operator_without_entries(gpu):
     st = tr.prepare(x)
     assert st.assembly['total_nnz'] == 0
     assert all(int(m.row_ptr[-1]) == 0 and m.row_ptr.numel() == m.rows + 1 for m in st.gather + st.spread)
+
+
+def test_scratch_of_few_point_cells(gpu):
+    """The chunk lists follow the points per cell: for 4-point tetrahedra they
+    take 96 bytes per cell, a twelfth of the stencil tables' 1152."""
+    X, cells = ofe.box_tets(20, (.3, .35, .4), (.7, .65, .75))
+    g = ofe.p1_solid(X, cells)
+    t = lambda a, dtype=torch.float64: torch.tensor(np.ascontiguousarray(a), device=gpu, dtype=dtype)
+    geometry, x = FEGeometry(t(g.cells, torch.int64), t(g.values), t(g.weights), len(X)), t(X)
+    grid = MACGrid((32, 32, 32), (1., 1., 1.))
+    tr = AssembledTransfer(grid, geometry)
+    stencil = from_points(tr.interaction_points(x), grid)
+    sizes = []
+    call = _abi.call
+
+    def counting(name, *args):
+        if name == 'afsi_p1_row_boxes_f64':
+            sizes.append(torch.cuda.memory_allocated() - base)
+        call(name, *args)
+
+    E, N = len(g.cells), len(X)
+    _abi.call = counting
+    try:
+        torch.cuda.synchronize()
+        base = torch.cuda.memory_allocated()
+        assert tr._rows(stencil.base, stencil.phi) is not None
+    finally:
+        _abi.call = call
+    # boxes of cells (72 B) and rows (72 B), two int64 per row and component, the chunk lists; 512 B per allocation
+    assert sizes[0] <= E * (72 + 96) + N * (72 + 48) + 6 * 512
