@@ -370,7 +370,9 @@ int check_rows(const afsi_fe_geometry* g, const afsi_grid3* grid) {
                      g->elements > 0 && g->node_count > 0,
                  "row assembly takes cells of at most 4 nodes and 64 points");
     AFSI_REQUIRE(!grid->periodic, "the assembled operator requires a closed MAC box");
-    AFSI_REQUIRE(g->elements < (int64_t(1) << 28) && g->node_count < (int64_t(1) << 28), "mesh too large for row assembly");
+    // a wave per row, and a launch takes fewer than 2^32 threads
+    AFSI_REQUIRE(g->elements < (int64_t(1) << 28) && WAVE * (3 * g->node_count + 7) < (int64_t(1) << 32),
+                 "mesh too large for row assembly");
     return OK;
 }
 

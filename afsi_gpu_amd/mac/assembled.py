@@ -173,7 +173,8 @@ class AssembledTransfer(FETransfer):
         shapes = [self.grid.face_shape(c) for c in range(3)]
         faces = [prod(shape) for shape in shapes]
         limit = _abi.load().afsi_p1_row_sites_limit()
-        if Q > 64 or sum(faces) >= 2 ** 31 - 3 or max(E, N) >= 2 ** 28:
+        # a wave per row: a launch takes fewer than 2^32 threads
+        if Q > 64 or sum(faces) >= 2 ** 31 - 3 or E >= 2 ** 28 or 64 * (3 * N + 7) >= 2 ** 32:
             return None
         grid, device = self.grid.abi(), g.weights.device
         empty = lambda *shape, dtype=torch.int32: torch.empty(shape, dtype=dtype, device=device)
