@@ -182,11 +182,17 @@ __global__ void __launch_bounds__(256) csr_spmv_kernel(afsi_csr a, const double*
 }
 
 // Rows of the gather matrix hold the hundreds of faces around a node, rows of
-// the spread matrix the few nodes around a face. A wave per row from 64
-// entries on average, where every lane has work: 4185 rows of hundreds take
-// 12 us against 67 with 8 lanes, which fill two waves per CU; 900000 short
-// rows take 23 us with 8 lanes.
-constexpr int64_t SPMV_LONG = 64;
+// the spread matrix the few nodes around a face. A wave per row where 8 lanes
+// per row leave the chip idle, up to 10240 rows (5 waves per CU) of at least
+// 64 entries, and where rows are long, which is at fewer entries
+// with very many rows. us by rows x entries, 8 lanes / a wave:
+//   4096 x 64: 7.0 / 7.8, x 256: 7.8 / 7.6; 6144 x 768: 41 / 13
+//   8192 x 256: 15.0 / 8.2; 10240 x 192: 12.5 / 9.8
+//   12288 x 128: 8.2 / 8.8, x 320: 22.7 / 14.8
+//   65536 x 112: 24 / 33, x 256: 45 / 53, x 320: 63 / 62, x 768: 194 / 145
+//   200000 x 128: 92 / 96, x 160: 130 / 121, x 320: 265 / 198
+constexpr int64_t SPMV_FEW_ROWS = 10240, SPMV_MANY_ROWS = 1 << 17;
+inline int64_t spmv_wave_from(int64_t rows) { return rows <= SPMV_FEW_ROWS ? 64 : (rows < SPMV_MANY_ROWS ? 320 : 160); }
 
 int check_table(const afsi_hash_table* t) {
     AFSI_REQUIRE(t && t->keys && t->values && t->flag, "null hash table");
@@ -242,7 +248,7 @@ int afsi_csr_spmv_f64(const afsi_csr* a, const double* x, int64_t x_stride, doub
                       double scale, void* stream) {
     AFSI_REQUIRE(a && a->row_ptr && a->cols && a->vals && x && y && a->rows > 0, "invalid CSR product arguments");
     AFSI_REQUIRE(x_stride >= 1 && y_stride >= 1, "CSR product strides must be positive");
-    if (a->nnz >= SPMV_LONG * a->rows)
+    if (a->nnz >= spmv_wave_from(a->rows) * a->rows)
         csr_spmv_kernel<WAVE><<<grid_for(a->rows * WAVE, 256, 16384), 256, 0, hipStream_t(stream)>>>(
             *a, x, x_stride, y, y_stride, scale);
     else

@@ -10,8 +10,8 @@ import torch
 from oracle import assembled as oas
 from oracle import fe as ofe
 from oracle import ib3d
-from afsi_gpu_amd.mac.assembled import AssembledTransfer, HashWorkspace, accumulate, sorted_entries
-from afsi_gpu_amd.mac.fe import FEGeometry, FETransfer
+from afsi_gpu_amd.mac.assembled import AssembledTransfer, HashWorkspace, accumulate, csr_apply, sorted_entries
+from afsi_gpu_amd.mac.fe import CSRMatrix, FEGeometry, FETransfer
 from afsi_gpu_amd.mac.grid import MACGrid
 
 pytestmark = pytest.mark.gpu
@@ -170,3 +170,24 @@ def test_dropin_contract_and_hash_accumulate(gpu):
         assert torch.equal(k2, keys) and torch.equal(v2, 2 * vals)
     with pytest.raises(NotImplementedError):
         cuda_ib.contract(stencil, groups[0], 0, 0, low, width, prefix, 0, grid.face_shape(0), work, cache=object())
+
+
+# either side of the lines between 8 lanes and a wave per row
+@pytest.mark.parametrize('rows,mean', [(1, 64), (7, 63), (10240, 64), (10241, 64), (10241, 319), (10241, 320),
+                                       (131072, 159), (131072, 160)])
+def test_csr_product_of_uneven_rows(gpu, rows, mean):
+    gen = np.random.default_rng(17)
+    counts = gen.integers(0, 2 * mean, size=rows)
+    counts[-1] = max(0, counts[-1] + mean * rows - counts.sum())  # at least the mean
+    ptr = np.concatenate(([0], np.cumsum(counts)))
+    cols = gen.integers(0, 5000, size=ptr[-1])
+    vals, x = gen.normal(size=ptr[-1]), gen.normal(size=(5000, 2))
+    A = CSRMatrix(t(ptr, gpu, torch.int32), t(cols, gpu, torch.int32), t(vals, gpu), rows)
+    y = torch.full((rows, 3), 7., device=gpu, dtype=torch.float64)
+    xs = t(x, gpu)
+    csr_apply(A, xs[:, 1], 2, y[:, 2], 3, .5)
+    terms = np.concatenate((vals * x[cols, 1], [0.]))
+    want, size = (np.add.reduceat(v, ptr[:-1]) * (counts > 0) for v in (terms, abs(terms)))
+    # two orders of a row's sum differ by at most its length in roundings of the sum of magnitudes
+    assert (abs(y[:, 2].cpu().numpy() - .5 * want) <= counts.max() * 2.3e-16 * size + 1e-300).all()
+    assert bool((y[:, :2] == 7).all())
