@@ -60,9 +60,10 @@ __host__ __device__ inline int stage_tiles(const Dim32& d, int tx, int ty) {
     return ((d.n0 + tx - 1) / tx) * ((d.n1 + ty - 1) / ty) * ((d.n2 + TILE_Z - 1) / TILE_Z);
 }
 
+// Two cells loaded or stored at once, at any address that one cell may have.
 template <class T> struct Pair2;
-template <> struct Pair2<float> { using type = float2; };
-template <> struct Pair2<double> { using type = double2; };
+template <> struct Pair2<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
+template <> struct Pair2<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
 
 // g wrapped into [0, n): one addition where the axis is longer than a halo.
 __device__ inline int wrap_near(int g, int n) {

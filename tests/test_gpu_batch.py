@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from afsi_gpu_amd import workloads
-from afsi_gpu_amd.batch import BatchedIBStep, BatchedMixedMultigrid
+from afsi_gpu_amd.batch import BatchedIBStep, BatchedMixedMultigrid, MixedState
 from afsi_gpu_amd.mac import MACGrid, MGOptions, MixedMultigrid
 from afsi_gpu_amd.step import IBStep
 
@@ -153,3 +153,28 @@ def test_batched_transfer_matches_per_instance(gpu, periodic):
         assert rel(outs[i], U) < 1e-12
         pbeg += x.shape[0]
         kbeg += ks
+
+
+@pytest.mark.parametrize('periodic', [True, False])
+def test_coarser_levels_at_any_float_address(gpu, periodic):
+    """A batch takes level buffers at any address of a float: the stages' pair
+    accesses ask for no more."""
+    grids = [MACGrid(s, (1., 1., 1.), periodic=periodic) for s in ((64, 64, 64), (64, 32, 48))]
+    options = MGOptions(smooth=2, smoother='rbgs')
+    rhs = [rhs_for(g.shape, i, gpu) for i, g in enumerate(grids)]
+    out = []
+    for shift in (0, 1):
+        states = [MixedState(g, device=gpu, options=options) for g in grids]
+        keep = []
+        for st in states:
+            mg = st.inner
+            for buffers in (mg.p, mg.rhs, mg.tmp):
+                for l in range(1, len(mg.shapes)):
+                    n = buffers[l].numel()
+                    keep.append(torch.zeros(n + shift, device=gpu, dtype=torch.float32))
+                    buffers[l] = keep[-1][shift:].view(mg.shapes[l])
+            zero_initial = mg.plan.zero_initial
+            mg.plan = mg._make_plan()
+            mg.plan.zero_initial = zero_initial
+        out.append(BatchedMixedMultigrid(states=states, device=gpu, options=options, graphs=False).solve(rhs)[0])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
