@@ -19,6 +19,13 @@ from oracle.mac3d import MGOptions as OOptions
 pytestmark = pytest.mark.gpu
 
 
+def close(got, want, bound):
+    """In the 2-norm, and cell by cell against the largest value (a few wrong
+    cells at a tile's edge would vanish in the norm)."""
+    assert np.linalg.norm(got - want) < bound * np.linalg.norm(want)
+    assert abs(got - want).max() < bound * abs(want).max()
+
+
 @pytest.mark.parametrize('periodic', [False, True], ids=['closed', 'periodic'])
 @pytest.mark.parametrize('smoother,nu', [('rbgs', 2), ('rbgs', 5), ('jacobi', 4), ('jacobi', 9)])
 @pytest.mark.parametrize('shape', [(24, 20), (128, 32), (160, 32), (192, 48), (72, 120), (512, 64)])
@@ -32,14 +39,18 @@ def test_cycle_matches_oracle(gpu, shape, smoother, nu, periodic):
     if periodic:
         p, rhs = p - p.mean(), rhs - rhs.mean()
     want = ref.cycle(0, p, rhs)
+    # A cell's residual is rounded to some eps diag |p|, and the coarse levels return that as errors of p as
+    # large as their smallest eigenvalue is small: smallest in a long closed channel, whose only fixed value is
+    # the outlet's. Measured: at most 1.8e-13 (FP32: 5.9e-5) closed and 1.9e-14 (1.1e-5) periodic, about half
+    # the bound.
+    bound = 4e-14 if periodic else 4e-13
     got = mg.cycle(torch.tensor(p, device=gpu), torch.tensor(rhs, device=gpu)).cpu().numpy()
-    # the cycle's own bound: about 50 FP64 roundings along any path of a contraction
-    assert np.linalg.norm(got - want) < 1e-12 * np.linalg.norm(want)
+    close(got, want, bound)
     single = ChannelMultigrid(grid, device=gpu, dtype=torch.float32,
                               options=MGOptions(smooth=nu, smoother=smoother), backend='workspace')
     got = single.cycle(torch.tensor(p, device=gpu, dtype=torch.float32),
                        torch.tensor(rhs, device=gpu, dtype=torch.float32)).double().cpu().numpy()
-    assert np.linalg.norm(got - want) < 1e-12 * 2. ** 29 * np.linalg.norm(want)  # the same bound in FP32
+    close(got, want, bound * 2. ** 29)  # FP32 rounds 2^29 times as coarsely
 
 
 def test_one_level(gpu):
@@ -49,7 +60,7 @@ def test_one_level(gpu):
     got = mg.cycle(torch.zeros((9, 5), device=gpu, dtype=torch.float64), torch.tensor(rhs, device=gpu)).cpu().numpy()
     ref = mac2d.ChannelMultigrid((9, 5), grid.spacing, OOptions(), False)
     want = ref.cycle(0, np.zeros((9, 5)), rhs)
-    assert np.linalg.norm(got - want) < 1e-12 * np.linalg.norm(want)
+    close(got, want, 4e-13)
 
 
 # Closed and periodic; the whole hierarchy in the tail, and one tiled level.
@@ -97,11 +108,14 @@ def test_periodic_cycle_of_a_rhs_with_a_mean(gpu, shape, smoother, nu):
     gen = np.random.default_rng(12)
     p, rhs = gen.normal(size=shape) + .7, gen.normal(size=shape) + 3.
     want = ref.cycle(0, p, rhs)
-    for dtype, bound in ((torch.float64, 1e-12), (torch.float32, 1e-12 * 2. ** 29)):
+    # as for the cycles above, on larger grids (the smallest eigenvalue falls with the square of the cells along
+    # the channel) and with residuals four times as large, a mean of 3 on values of 1: measured 5.3e-14 in FP64
+    tight = 2e-13
+    for dtype, bound in ((torch.float64, tight), (torch.float32, tight * 2. ** 29)):
         mg = ChannelMultigrid(grid, device=gpu, dtype=dtype, options=MGOptions(smooth=nu, smoother=smoother),
                               backend='workspace')
         got = mg.cycle(torch.tensor(p, device=gpu, dtype=dtype), torch.tensor(rhs, device=gpu, dtype=dtype))
-        assert np.linalg.norm(got.double().cpu().numpy() - want) < bound * np.linalg.norm(want)
+        close(got.double().cpu().numpy(), want, bound)
     other = ChannelGrid((32, 16), (2., 1.), False)
     batch = BatchedChannelStep([other, grid], [1, 1], dt=1e-3, device=gpu,
                                options=MGOptions(smooth=nu, smoother=smoother))
@@ -109,4 +123,4 @@ def test_periodic_cycle_of_a_rhs_with_a_mean(gpu, shape, smoother, nu):
     solver.p[0].copy_(torch.tensor(p))
     solver.rhs[0].copy_(torch.tensor(rhs))
     _abi.call('afsi_chb_cycles_f64', byref(batch.batch), None, 1, _abi.stream())
-    assert np.linalg.norm(solver.p[0].cpu().numpy() - want) < 1e-12 * np.linalg.norm(want)
+    close(solver.p[0].cpu().numpy(), want, tight)

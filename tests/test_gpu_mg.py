@@ -225,8 +225,9 @@ def test_projection_matches_oracle(gpu, periodic):
 
 
 def test_autotuned_sweeps_keep_results(gpu):
-    """Tuned tile/grid choices change only speed: a tuned solve equals the
-    default one bit for bit."""
+    """Tuned tile/grid choices change only speed: a solve with tuned sweeps
+    (levels untiled, so that the cycle runs them) equals the default one bit
+    for bit."""
     from afsi_gpu_amd import autotune
     grid = MACGrid((64, 64, 64), (1., 1., 1.), periodic=True)
     opts = MGOptions(smooth=2, smoother='rbgs')
@@ -235,8 +236,10 @@ def test_autotuned_sweeps_keep_results(gpu):
     rhs -= rhs.mean()
     b = torch.tensor(rhs, device=gpu)
     ref = GeometricMultigrid(grid, device=gpu, options=opts, backend='workspace')
+    ref.plan.fuse_cells = -1
     p0, i0 = ref.solve(b)
     tuned = GeometricMultigrid(grid, device=gpu, options=opts, backend='workspace')
+    tuned.plan.fuse_cells = -1
     chosen = autotune.tune_sweeps(tuned)
     assert 0 in chosen and chosen[0][0] in (2, 4)
     p1, i1 = tuned.solve(b)

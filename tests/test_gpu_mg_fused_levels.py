@@ -1,12 +1,12 @@
-"""Fused small multigrid levels (vdown_kernel: two red-black sweeps, the
-residual and its restriction in one launch; vup_kernel: the prolongation
-and two sweeps in another) against the same driver with every level
-unfused (plan.fuse_cells = -1), and against the oracle.
+"""Tiled smoothing stages (stage_kernel: a few half-sweeps of a tile in one
+launch, with the restricted residual after the last one down and the
+prolongation before the first one up) against the same driver with every
+level untiled (plan.fuse_cells = -1), and against the oracle.
 
-The fused kernels form every value with the expressions and summation order
-of the unfused sweep, restriction and prolongation kernels, and the library
-is compiled without floating-point contraction, so the two drivers must
-agree bit for bit; the oracle comparison pins both."""
+For red-black levels with an even z extent up to 128 the two form every value
+with the same expressions and summation order, and the library is compiled
+without implicit floating-point contraction, so they must agree bit for bit;
+the oracle comparison pins both."""
 from math import pi
 
 import numpy as np
@@ -40,10 +40,9 @@ def solver(gpu, shape, periodic, dtype, fuse):
     return mg
 
 
-def fused_levels(shapes):
-    """Levels the driver fuses by default (z extent 32/64, <= 64^3 cells,
-    above the LDS coarse levels)."""
-    return [s for s in shapes[:-1] if s[2] in (32, 64) and np.prod(s) <= 64 ** 3 and np.prod(s) > 4096]
+def tiled_levels(shapes):
+    """Levels the driver tiles by default: those above the LDS coarse levels."""
+    return [s for s in shapes[:-1] if np.prod(s) > 4096]
 
 
 @pytest.mark.parametrize('dtype', [torch.float64, torch.float32])
@@ -54,7 +53,7 @@ def test_fused_levels_match_unfused_bitwise(gpu, shape, periodic, dtype):
     out = []
     for fuse in (True, False):
         mg = solver(gpu, shape, periodic, dtype, fuse)
-        assert fused_levels(mg.shapes), 'shape reaches no fused level'
+        assert tiled_levels(mg.shapes), 'shape reaches no tiled level'
         mg.initialize(torch.tensor(start, device=gpu, dtype=dtype), torch.tensor(rhs, device=gpu, dtype=dtype))
         for _ in range(3):
             mg._cycles(1)
@@ -85,7 +84,7 @@ def test_fused_cycle_matches_oracle(gpu, shape, periodic, dtype):
 @pytest.mark.parametrize('periodic', [False, True])
 def test_mixed_solve_fused_matches_unfused(gpu, periodic):
     """The mixed solve's FP32 cycles start from a zero iterate
-    (zero_initial): the fused down kernel then reads no p at level 0."""
+    (zero_initial): the first stage then reads no p at level 0."""
     shape = (64, 64, 64)
     _, rhs, _ = manufactured(shape, periodic)
     results = []

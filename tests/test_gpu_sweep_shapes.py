@@ -1,8 +1,9 @@
-"""The red-black sweep specialisations the 128^3 and 64^3 levels run
+"""The red-black sweep specialisations of untiled 128^3 and 64^3 levels
 (rb_rows_kernel with the z extent 128 or 64 as a compile-time constant, for
 2x2, 4x4, 8x4 and 8x8 row tiles) against the oracle, on small grids whose
 levels reach them: (32, 32, 128) and (16, 16, 64), both boundary types, FP64
-and FP32. One V(2,2) cycle from a manufactured start, then the per-cycle
+and FP32. The plan keeps its levels untiled (fuse_cells = -1): tiled smoothing
+stages would take their place. One V(2,2) cycle from a manufactured start, then the per-cycle
 residual reduction of a solve (FP64 within 1e-10 of the oracle's, same cycle
 count; FP32 cycles within FP32 rounding of the FP64 oracle cycle)."""
 from math import pi
@@ -28,10 +29,11 @@ def manufactured(shape):
     return h, exact - exact.mean()
 
 
-def solver(gpu, shape, periodic, tile, dtype, check_every=2, relax=1.):
+def solver(gpu, shape, periodic, tile, dtype, check_every=2, relax=1., fuse_cells=-1):
     mg = GeometricMultigrid(MACGrid(shape, LENGTHS, periodic=periodic), device=gpu, dtype=dtype,
                             options=MGOptions(smooth=2, smoother='rbgs', check_every=check_every, relax=relax),
                             backend='workspace')
+    mg.plan.fuse_cells = fuse_cells
     for level, s in enumerate(mg.shapes):
         tx, ty = TILES[tile]
         if s[0] % tx == 0 and s[1] % ty == 0:
@@ -81,10 +83,11 @@ def test_solve_history_with_forced_sweep_tiles(gpu, shape, periodic, tile):
 @pytest.mark.parametrize('dtype', [torch.float64, torch.float32])
 @pytest.mark.parametrize('periodic', [False, True])
 @pytest.mark.parametrize('shape', [(32, 32, 128), (16, 16, 64)])
-def test_over_relaxed_red_black(gpu, shape, periodic, dtype):
+@pytest.mark.parametrize('fuse_cells', [-1, 0], ids=['sweeps', 'stages'])
+def test_over_relaxed_red_black(gpu, shape, periodic, dtype, fuse_cells):
     """Over-relaxed red-black smoothing (relax 1.3) on every level kind the
-    fused driver has (row sweeps at z 128/64, fused small levels, the LDS
-    coarse cycle): one cycle against the oracle's over-relaxed cycle, and in
+    fused driver has (row sweeps at z 128/64, tiled stages, the LDS coarse
+    cycle): one cycle against the oracle's over-relaxed cycle, and in
     FP64 the per-cycle residual reduction of a solve within 1e-10 with the
     same (smaller) cycle count."""
     relax = 1.3
@@ -95,7 +98,7 @@ def test_over_relaxed_red_black(gpu, shape, periodic, dtype):
     start -= start.mean()
     ref = mac3d.Multigrid(shape, h, mac3d.MGOptions(smooth=2, smoother='rbgs', relax=relax), periodic)
     expected = ref.cycle(0, start, rhs)
-    mg = solver(gpu, shape, periodic, 4, dtype, relax=relax)
+    mg = solver(gpu, shape, periodic, 4, dtype, relax=relax, fuse_cells=fuse_cells)
     mg.initialize(torch.tensor(start, device=gpu, dtype=dtype), torch.tensor(rhs, device=gpu, dtype=dtype))
     got = mg.cycle().double().cpu().numpy()
     got -= got.mean()
@@ -108,7 +111,7 @@ def test_over_relaxed_red_black(gpu, shape, periodic, dtype):
     _, info_ref = ref.solve(rhs)
     plain = mac3d.Multigrid(shape, h, mac3d.MGOptions(smooth=2, smoother='rbgs', check_every=1), periodic)
     _, info_plain = plain.solve(rhs)
-    mg = solver(gpu, shape, periodic, 4, torch.float64, check_every=1, relax=relax)
+    mg = solver(gpu, shape, periodic, 4, torch.float64, check_every=1, relax=relax, fuse_cells=fuse_cells)
     hist = []
     mg.solve(torch.tensor(rhs, device=gpu), history=hist)
     rho = np.array(hist) / hist[0]
