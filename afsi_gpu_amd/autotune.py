@@ -3,7 +3,9 @@
 * Red-black sweeps: per multigrid level, the tile (2x2, 4x4, 8x4 or 8x8
   rows) and the
   persistent grid size (one tile per workgroup, or fewer workgroups that
-  pipeline several tiles each). Every variant computes the same values
+  pipeline several tiles each). These are the launches of untiled levels
+  (``plan.fuse_cells`` negative or smaller than the level); by default the
+  V-cycle runs tiled smoothing stages, which the tuned values do not change. Every variant computes the same values
   (the per-cell arithmetic does not depend on the tiling), so tuning only
   changes speed. Cached by (level shape, dtype, boundary type).
 * Transfer tile: the binning/spread/interpolation tile edge (4 or 8 cells)
@@ -38,7 +40,8 @@ def _time(fn, repeats):
 
 def tune_sweeps(solver, repeats=20):
     """Choose sweep_tile / sweep_blocks for every level of a fused
-    ``GeometricMultigrid`` (red-black) and write them into its plan.
+    ``GeometricMultigrid`` (red-black) and write them into its plan; they
+    take effect on levels that the plan leaves untiled (``fuse_cells``).
     Returns {level: (tile, blocks, microseconds)}."""
     if not solver.fused or solver.options.smoother != 'rbgs':
         return {}

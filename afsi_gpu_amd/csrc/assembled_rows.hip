@@ -20,8 +20,9 @@
 // one tap per lane: 4 LDS reads and 2 products per lane for 256 tap products
 // instead of 12 and 8. The lane's site gets one LDS add per four points.
 //
-// Bound: instruction issue of one wave per row (some 20 per chunk of four
-// points), as many rows per CU as their boxes leave room for. 16200 cells of
+// Bound: the chain of one wave per row (some 20 instructions per chunk of four
+// points; VALU issue takes 0.21 of the time with 1.4 waves per SIMD), as many
+// rows per CU as their boxes leave room for. 16200 cells of
 // 64 points, 4185 nodes, 96^3 faces: all three matrices and transposes 0.93
 // ms against 6.83 ms through the table; rows_kernel 427 us, against 785 us
 // with the chunks found per node instead of once per cell, the site read and
@@ -40,8 +41,11 @@ constexpr int UNROLL = 4;              // chunks whose operands are read togethe
 // Chunk slots per cell: a cell of Q points has at most Q chunks.
 __host__ __device__ inline int chunk_slots(int quad) { return (quad + UNROLL - 1) / UNROLL * UNROLL; }
 // What LDS holds: 128 KB of sites + 6.6 KB of points. Rows beat the table
-// wherever they fit: 0.28 / 2.78 ms for 468 nodes with rows up to 1320
-// sites, 0.34 / 5.12 ms up to 3808, 0.65 / 7.23 ms up to about 12000.
+// wherever they fit. 64 points per cell: 0.28 / 2.78 ms for 468 nodes with
+// rows up to 1320 sites, 0.34 / 5.12 ms up to 3808, 0.65 / 7.23 ms up to about
+// 12000. Whole preparations with 4 points per tetrahedron: 0.46 / 2.12 ms for
+// 384 cells on 32^3, 0.88 / 6.14 ms for 48000; with 3 per triangle: 0.66 /
+// 4.20 ms for 20480.
 constexpr int64_t ROW_SITES = 16384;
 
 struct RowStats {  // int64 words, zeroed by the caller

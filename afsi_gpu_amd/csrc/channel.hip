@@ -9,10 +9,12 @@
 //   P = true   periodic in x, walls in y (build-own); singular, so the
 //              driver removes means as the 3D closed box does
 //              (mac/multigrid.py:107-123).
-// Cell (x, y) of an nx x ny level is element x*ny + y. Every elementwise
-// kernel evaluates the reference's expression in the reference's order
-// (mac2d/_triton_mg.py:7-75), so results are bit-identical to the
-// restatement in FP64 (compiled with -ffp-contract=off).
+// Cell (x, y) of an nx x ny level is element x*ny + y. The elementwise entry
+// points (stencil, divergence, correction, single sweeps, restriction,
+// prolongation) evaluate the reference's expression in the reference's order
+// (mac2d/_triton_mg.py:7-75), so they are bit-identical to the restatement in
+// FP64 (compiled with -ffp-contract=off). The V-cycle's smoothing has its own
+// expressions (channel_vcycle.hpp) and agrees with it within rounding.
 #include "binshare.hpp"
 #include <algorithm>
 #include <cstring>
@@ -482,11 +484,11 @@ static int channel_tail(const afsi_mg2d_plan& pl, int l0, int cycles, size_t byt
 
 // V-cycles: the levels whose hierarchy does not fit one workgroup's LDS
 // (chf_split) as tiled launches, one per smoothing stage of up to CHF_MAX
-// phases, the rest in the tail. Measured per red-black V(2,2) cycle (FP64,
-// periodic, kernel time): 256x64 32 us (two tile launches of 5.4 us around a
-// 21.7 us tail) against 166 us with every phase on global memory in one
-// workgroup; 128x32 whole in the tail 16.4 us against 90 us. Jacobi V(4,4)
-// 512x128: 53 us in five launches against 135 us in 52. The line between
+// phases, the rest in the tail. Measured for two FP64 cycles and a residual:
+// periodic red-black V(2,2) at 256x64 92 us (tile launches of 5.5 us around a
+// 22.6 us tail) against 338 us with every phase on global memory in one
+// workgroup, 128x32 whole in the tail 56 against 142 us; closed Jacobi V(4,4)
+// at 512x128 116 us against 252 us in one launch per phase. The line between
 // the two forms is the LDS: a level that fits costs 3-8 us in the tail, which
 // is less than two launches and their gaps.
 template <class T>

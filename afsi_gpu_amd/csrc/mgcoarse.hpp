@@ -8,10 +8,13 @@
 // black cells of a level are separate arrays indexed by pair, so lanes read
 // consecutive words and a cell's neighbours are all in the other colour's
 // array (the pair's own neighbour is a register). A missing neighbour is a
-// word of zeros behind the array. Kernel time of the 16^3 cycle with its 8^3
-// and 4^3 levels: FP32 red-black 21.0 -> 16.6 us, FP64 23.7 -> 18.8,
-// FP64 closed Jacobi V(4,4) 43 -> 23.6 (packed cell lists decoded per
-// update, colours interleaved in one array).
+// word of zeros behind the array (red-black) or the cell itself (Jacobi, whose
+// update is in difference form). Kernel time of the 16^3 cycle with its 8^3
+// and 4^3 levels: FP32 periodic red-black 21.0 -> 16.6 us, FP64 23.7 -> 17.9,
+// FP64 closed Jacobi V(4,4) 43 -> 24.7 (packed cell lists decoded per
+// update, colours interleaved in one array). Half to two thirds of the cycles
+// of its four SIMDs issue VALU instructions (0.55 of the Jacobi, 0.65 of the
+// FP32 kernel); the rest are barriers and LDS round trips.
 
 constexpr int COARSE_PAIRS = int(COARSE_MAX / 2 / COARSE_THREADS);  // z pairs per thread
 static_assert(COARSE_PAIRS * 2 * COARSE_THREADS == COARSE_MAX, "whole pairs per thread");

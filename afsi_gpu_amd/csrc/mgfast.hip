@@ -1293,12 +1293,21 @@ struct FastRunner {
     // where the level fills the chip several times over (redundant cells are
     // then the cost); smaller levels are bound by launches and by the length of
     // one workgroup's instruction stream, so they take four phases and, up to
-    // 256 (down) or below 256 (up) 8x8 tiles, the shorter 4x8 tile. Measured,
-    // periodic red-black, us per V(2,2) level visit (down + up):
-    //   FP32 128^3: 4 x 11-14 (two phases) 46, four phases 55, sweep kernels 56
-    //   FP64 128^3: 70, 89, 106
-    //   FP32 64^3: two phases 21 (and two more launches), 4x8 / 8x8 15
-    //   FP64 64^3: 21, 19; one fused launch per stage on full z rows took 40
+    // 256 (down) or below 256 (up) 8x8 tiles, the shorter 4x8 tile. Measured
+    // per V-cycle in us with level 0 in two phases / four on 4x8 / four on 8x8,
+    // V(2,2) red-black or V(4,4) Jacobi:
+    //             periodic RB FP64   periodic RB FP32   closed Jacobi FP64
+    //   48^3      56.3 47.4 53.8     49.4 41.7 45.0     76.9 67.1 76.0
+    //   64^3      60.8 58.3 59.0     53.0 50.4 50.1     82.2 81.8 81.7
+    //   80^3      92.1 80.2 85.3     73.5 62.9 67.3     126 118 132
+    //   96^3      93.9 98.6 96.3     74.2 73.7 72.2     141 155 179
+    //   112^3     178 159 168        138 121 122        241 239 285
+    //   128^3     136 158 144        102 112 103        221 265 299
+    // Over both boundary types, smoothers and precisions from 32^3 to 160^3 the
+    // rule is within 8% of the best of the three except where extents are no
+    // multiples of the tile (112^3 red-black: 4% to 17% behind 4x8) and for
+    // closed FP64 Jacobi from 80^3 to 112x96x96, whose 8x8 four-phase form
+    // runs out of registers (12% to 26% behind the best).
     static constexpr int64_t WIDE_TILES = 1024;
     bool wide(int l) const { return stage_tiles(D(l), 8, 8) >= WIDE_TILES; }
 
@@ -1325,8 +1334,7 @@ struct FastRunner {
             a.d = D(l);
             a.k = K(l);
             a.omega = T(pl.omega);
-            a.first = c * per;
-            a.count = phases - a.first < per ? phases - a.first : per;
+            a.count = std::min(per, phases - c * per);
             a.zero = zero && c == 0;
             const int r = pl.smoother == 1 ? stage_launch<true>(a, two, up) : stage_launch<false>(a, two, up);
             if (r) return r;
@@ -1495,7 +1503,7 @@ static int batch_layout(const afsi_mgb_batch* bt, BatchLayout& L) {
         for (int l = 0; l < L.cf[i]; ++l)
             AFSI_REQUIRE(pl.n[l][2] <= ZROW && pl.n[l][2] % 2 == 0 && pl.n[l][0] % 2 == 0 &&
                              pl.n[l][1] % 2 == 0,
-                         "instance %d level %d: batched sweeps need even extents and z <= %d", i, l, ZROW);
+                         "instance %d level %d: batched solves need even extents and z <= %d", i, l, ZROW);
         AFSI_REQUIRE(pl.n[0][0] * pl.n[0][1] * pl.n[0][2] < (int64_t(1) << 31), "instance too large");
         if (L.cf[i] > L.levels) L.levels = L.cf[i];
     }
@@ -1510,7 +1518,8 @@ static int batch_layout(const afsi_mgb_batch* bt, BatchLayout& L) {
             const int64_t* nn = bt->items[i].plan.n[l];
             tiles += stage_tiles(Dim32{int(nn[0]), int(nn[1]), int(nn[2])}, 8, 8);
         }
-        // the rule of FastRunner::wide and stage_launch over the whole level
+        // the rule of FastRunner::wide and stage_launch over the whole level, one
+        // tile for both directions
         L.phases[l] = tiles >= FastRunner<float>::WIDE_TILES ? 2 : 4;
         L.tile_x[l] = tiles < 256 ? 4 : 8;
         L.chunks[l] = (2 * L.nu + L.phases[l] - 1) / L.phases[l];
@@ -1589,8 +1598,7 @@ static int batch_prepare(const afsi_mgb_batch* bt, hipStream_t s) {
                 a.out = buffers[1 - (c & 1)];
                 a.coarse = up && k == 0 ? static_cast<const float*>(pl.p[l + 1]) : nullptr;
                 a.restricted = !up && k == L.chunks[l] - 1 ? static_cast<float*>(pl.rhs[l + 1]) : nullptr;
-                a.first = k * L.phases[l];
-                a.count = std::min(L.phases[l], 2 * L.nu - a.first);
+                a.count = std::min(L.phases[l], 2 * L.nu - k * L.phases[l]);
                 a.zero = c == 0;  // a cycle starts from zero
                 descs[size_t(c) * m + j] = StageDesc{a, bt->active + i, begin};
                 if (c == 0) {  // except on level 0 of a later cycle of one refinement iteration

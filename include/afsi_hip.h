@@ -337,11 +337,13 @@ typedef struct afsi_mg3d_plan {
 int afsi_mg3d_supported(const afsi_mg3d_plan* plan);
 /* Doubles of reduce_partials the fused driver needs for level-0 extent n. */
 int64_t afsi_mg3d_partials_doubles(const int64_t n[3]);
-/* Fused driver (the production path). Per fine level: nu single-launch
- * sweeps (red-black: LDS tile + 2-cell halo, red on tile+1 ring then
- * black; or weighted Jacobi), one residual-restriction, one prolongation;
- * levels selected by fuse_cells instead run their smoothing stages tiled
- * (red-black: with identical results).
+/* Fused driver (the production path). Fine levels run their smoothing
+ * stages tiled, two or four phases (half-sweeps or Jacobi sweeps) per launch.
+ * Levels above fuse_cells, with planes of 2^28 cells or with buffers that are
+ * not aligned to 16 bytes run nu single-launch sweeps instead (red-black:
+ * LDS tile + 2-cell halo, red on tile+1 ring then black; or weighted
+ * Jacobi), one residual-restriction and one prolongation. The two agree bit
+ * for bit for red-black on even z extents up to 128, else within rounding.
  * All levels with <= 4096 cells run as one 1024-thread workgroup out of
  * LDS (including the dense coarse solve). No level performs the
  * reference's intermediate mean subtractions (mac/multigrid.py:107-123):
@@ -354,8 +356,8 @@ int afsi_mg3d_cycles_f32(const afsi_mg3d_plan* plan, int32_t cycles, void* strea
  * rhs[0] - A p[0] (two launches, no grid-wide synchronisation). */
 int afsi_mg3d_residual_f64(const afsi_mg3d_plan* plan, void* stream);
 int afsi_mg3d_residual_f32(const afsi_mg3d_plan* plan, void* stream);
-/* One smoothing sweep of `level` from p[level] into tmp[level] (exactly
- * the kernel the fused driver launches there); for timing. */
+/* One smoothing sweep of `level` from p[level] into tmp[level]: the kernel
+ * that the fused driver launches where the level is not tiled; for timing. */
 int afsi_mg3d_sweep_f64(const afsi_mg3d_plan* plan, int32_t level, void* stream);
 int afsi_mg3d_sweep_f32(const afsi_mg3d_plan* plan, int32_t level, void* stream);
 /* FP64 iterative refinement around FP32 V-cycles (build-own mixed
