@@ -951,6 +951,8 @@ struct VecDesc {
 
 constexpr int VEC_CHUNK = 4096;  // elements per workgroup in batched vector passes
 
+// The stage of every instance that has the level, tiles in the order of the
+// instances (not dealt to the XCDs in runs as in stage_kernel).
 template <bool P, int TX, int NPH, bool RESTRICT>
 __global__ void __launch_bounds__((Tile3<float, TX, 8, NPH, RESTRICT>::NT)) stage_batch_kernel(
     const StageDesc* __restrict__ desc, int n) {

@@ -8,7 +8,7 @@
 // of every x plane of its column: both values, both right-hand sides of all
 // planes stay in registers, so x neighbours and the pair's own neighbour are
 // registers, and only y and outer z neighbours go through LDS: an update is
-// three LDS reads, seven (Gauss-Seidel) or thirteen (Jacobi) floating-point
+// three LDS reads, eight (Gauss-Seidel) or thirteen (Jacobi) floating-point
 // operations and one LDS write. Jacobi updates in difference form,
 // p + omega (b - sum w (p - nb)) / diag, as the unfused sweeps do: from
 // (b + sum w nb) / diag the residual stagnates 1.6 to 1.8 times higher.
